@@ -19,9 +19,10 @@ Planes per kind: 0 (GPTQ) Xᵀ; 1 (GPTAQ) Xᵀ and the bf16 hi/lo parts of
 s[t,g]·(1/T_b), from which the Gram kernel forms x·s itself.  Activations
 that are not bf16 take P bf16 planes for Xᵀ that sum to it exactly (fp16: 2,
 fp32: 3; the reference's ``inp.float()``, gptq_utils.py:125), and the
-weighted kind then stages the hi/lo parts of (x·s[t,g])ᵀ as planes: every
-Gram product runs once per plane of its column operand (four, resp. nine
-times the bf16 Gram work for GPTQ).  The library gives each layout's height
+weighted kind then stages the hi/lo parts of (x·s[t,g])ᵀ as planes; a Gram
+product sums over the pairs of its operands' planes.  GPTQ's fp16 activations
+are staged and multiplied as fp16, one product as for bf16.
+The library gives each layout's height
 (``g2ptq_hessian_stage_height``).
 
 The first buffer holds 32 batches of the first batch's size (at least 65536

@@ -34,9 +34,10 @@
 //     bank-conflict free on 32- and 64-bank LDS.
 // K is split S ways when the tile grid alone would not fill the GPU: each
 // split writes its raw fp32 tile to a workspace and gram_reduce_kernel sums
-// the splits in a fixed order (deterministic) into the output.  A two-plane
-// (hi, lo) operand runs as a product over twice the tokens: the first half of
-// the splits multiplies hi against Xᵀ, the second half lo against Xᵀ.
+// the splits in a fixed order (deterministic) into the output.  A product of
+// operands of several planes sums over pairs of planes ("parts"): an equal
+// share of the splits multiplies each pair, all in one launch (hi and lo
+// against Xᵀ for GPTAQ).
 #include <algorithm>
 
 #include "common.hpp"
@@ -45,6 +46,7 @@ namespace g2ptq {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int TT = 256;   // output tile edge
@@ -334,18 +336,21 @@ __global__ void zero_cols_bf16_kernel(uint16_t* XT, int64_t ldt, int64_t rows, i
     XT[(e / w) * ldt + k0 + (e % w)] = 0;
 }
 
+// Most plane pairs a product sums over (fp32 activations: kXParts below).
+constexpr int kMaxParts = 6;
+
 struct G2Args {
-  const uint16_t* A1;  // row operand planes (Cp × ldt): A2 feeds the second and
-  const uint16_t* A2;  // A3 the third part of the splits when halves is 2 or 3
-  const uint16_t* A3;
-  const uint16_t* B;   // column operand plane
+  // The product is Σ over `parts` pairs of planes (row operand A[p], column
+  // operand B[p], Cp × ldt each); part p feeds splits [p, p + 1)·S / parts.
+  const uint16_t* A[kMaxParts];
+  const uint16_t* B[kMaxParts];
   int64_t ldt;
   int64_t kc;      // tokens per split (an even number of KS stages)
   int64_t nt;      // tiles per dimension
   int64_t tiles;   // upper triangle nt (nt + 1) / 2, or nt² for full products
   int64_t C;
-  int S;           // splits (halves × splits per half)
-  int halves;
+  int S;           // splits (parts × splits per part)
+  int parts;
   float alpha, beta;
   float* H; int64_t ldh;
   float* P;        // split partials: (tile * S + s) * TT*TT
@@ -503,7 +508,18 @@ __device__ __forceinline__ void store_tile(const G2Args& a, float* H, float* Pt,
   }
 }
 
-template <bool HAS_BETA, bool FULL>
+// One MFMA of 16 tokens: bf16 planes, or fp16 activations as they are (the
+// fp16 MFMA takes subnormal inputs at full value, measured on MI355X).
+template <bool F16>
+__device__ __forceinline__ f32x16 gram_mma(bf16x8 a, bf16x8 b, f32x16 c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+template <bool HAS_BETA, bool FULL, bool F16 = false>
 __global__ __launch_bounds__(NTH) void gram256_kernel(G2Args a) {
   __shared__ __attribute__((aligned(16))) uint16_t Ls[2][2][TT * KS];  // [buf][A/B]
 
@@ -530,12 +546,11 @@ __global__ __launch_bounds__(NTH) void gram256_kernel(G2Args a) {
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 2, wn = wave & 3;
 
-  // Split → operand plane and token range.
-  const int per_half = a.S / a.halves;
-  const int half = split / per_half, sp = split - half * per_half;
-  const uint16_t* Aop = half == 0 ? a.A1 : (half == 1 ? a.A2 : a.A3);
-  const uint16_t* Ag = Aop + (I * TT) * a.ldt + (int64_t)sp * a.kc;
-  const uint16_t* Bg = a.B + (J * TT) * a.ldt + (int64_t)sp * a.kc;
+  // Split → operand planes and token range.
+  const int per_part = a.S / a.parts;
+  const int part = split / per_part, sp = split - part * per_part;
+  const uint16_t* Ag = a.A[part] + (I * TT) * a.ldt + (int64_t)sp * a.kc;
+  const uint16_t* Bg = a.B[part] + (J * TT) * a.ldt + (int64_t)sp * a.kc;
 
   // Chunk q = tid + i*512 of a stage: row q >> 3, 16-byte chunk q & 7.
   // Two register sets carry stages kt+1 and kt+2 while stage kt is multiplied.
@@ -603,7 +618,7 @@ __global__ __launch_bounds__(NTH) void gram256_kernel(G2Args a) {
       }                                                                                 \
       _Pragma("unroll") for (int m = 0; m < 4; ++m)                                     \
       _Pragma("unroll") for (int n = 0; n < 2; ++n)                                     \
-        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[m], bv[n], acc[m][n], 0, 0, 0); \
+        acc[m][n] = gram_mma<F16>(av[m], bv[n], acc[m][n]);                            \
     }                                                                                   \
   } while (0)
 
@@ -728,8 +743,8 @@ __global__ __launch_bounds__(NTH) void wgram_kernel(G2Args a) {
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 2, wn = wave & 3;
 
-  const uint16_t* Ag = a.B + (I * TT) * a.ldt + (int64_t)split * a.kc;
-  const uint16_t* Bg = a.B + (J * TT) * a.ldt + (int64_t)split * a.kc;
+  const uint16_t* Ag = a.B[0] + (I * TT) * a.ldt + (int64_t)split * a.kc;
+  const uint16_t* Bg = a.B[0] + (J * TT) * a.ldt + (int64_t)split * a.kc;
   // Chunk q = tid + i*512 of a stage tile: row q >> 2, 16-byte chunk q & 3.
   const int qrow = tid >> 2, qc = tid & 3;  // chunk i adds 128 rows
   const float* Wg = a.W + grp * a.ldw + (int64_t)split * a.kc + qc * 8;
@@ -938,19 +953,21 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
   }
 }
 
-// Split plan.  Splits per operand half: the smallest power of two that gives
-// at least 4096 workgroups (16 waves of one 256×256 tile per CU), at most 16
-// splits in all and at least 16 KS-token stages per split; then, among the
+// Split plan.  Splits per part (pair of operand planes) of a product whose row
+// operand has `planes` planes: the smallest power of two that gives at least
+// 4096 workgroups (16 waves of one 256×256 tile per CU) for one column plane,
+// at most 16 splits of one column plane in all and at least 16 KS-token stages
+// per split; then, among the
 // counts down to three quarters of it, the one whose grid fills its last wave
 // of workgroups best (one workgroup per CU, kCUs of them): C=4096 has 136
 // tiles, 2176 workgroups (8.5 waves) at 16 splits and 2040 (7.97) at 15, and
 // its Gram takes 4.25 instead of 4.49 ms; C=14336 keeps 4 splits (6384
 // workgroups, 24.9 waves).  Measured on MI355X with random bf16 operands.
 // Every split gets an even number of stages, so the staged width is K padded
-// to a multiple of 2·KS·(splits per half), at most 2048.
+// to a multiple of 2·KS·(splits per part), at most 2048.
 struct GramPlan {
   int S;        // total splits
-  int64_t Kp;   // padded tokens per half
+  int64_t Kp;   // padded tokens per part
   int64_t kc;   // tokens per split
 };
 
@@ -959,23 +976,23 @@ constexpr int64_t kCUs = 256;  // MI355X
 // Share of the workgroup slots that a grid of n workgroups keeps busy over its waves.
 double wave_fill(int64_t n) { return (double)n / (double)(cdiv(n, kCUs) * kCUs); }
 
-GramPlan gram_plan(int64_t tiles, int64_t K, int halves, int64_t max_chain = 0,
+GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, int64_t max_chain = 0,
                    int64_t max_s = 16) {
   const int64_t K1 = std::max<int64_t>(K, 1);
   const int64_t smax =
-      std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(16 / halves, max_s), K1 / (KS * 16)));
+      std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(16 / planes, max_s), K1 / (KS * 16)));
   int s = 1;
-  while (s * 2 <= smax && tiles * halves * s < 4096) s *= 2;
+  while (s * 2 <= smax && tiles * planes * s < 4096) s *= 2;
   {
     int best = s;
     for (int c = s - 1; c >= 1 && 4 * c >= 3 * s; --c)
-      if (wave_fill(tiles * halves * c) > wave_fill(tiles * halves * best) + 1e-9) best = c;
+      if (wave_fill(tiles * planes * c) > wave_fill(tiles * planes * best) + 1e-9) best = c;
     s = best;
   }
   while (max_chain > 0 && s * 2 <= smax && cdiv(K1, s) > max_chain) s *= 2;
   const int64_t step = (int64_t)2 * KS * s;
   GramPlan p;
-  p.S = s * halves;
+  p.S = s * parts;
   p.Kp = cdiv(K1, step) * step;
   p.kc = p.Kp / s;
   return p;
@@ -990,35 +1007,62 @@ size_t plan_ws_bytes(int64_t tiles, const GramPlan& p) {
   return p.S == 1 ? 256 : (size_t)tiles * p.S * TT * TT * sizeof(float);
 }
 
-// The products, as (full, halves).
-struct Product {
-  bool full;
-  int halves;
-};
-constexpr Product SYM1{false, 1};  // H from Xᵀ
-constexpr Product SYM2{false, 2};  // weighted H[g] from (hi_g, lo_g) against Xᵀ
-constexpr Product FULL2{true, 2};  // GPTAQ Dx from (hi, lo) against Xᵀ
-
 // Staged bf16 planes of one activation: 1 for bf16, 2 for fp16, 3 for fp32
-// (dtype codes 0, 1, 2).  With P > 1 every product runs once per plane q of
-// the column operand (Σ_q planes = X), accumulating into the output, and the
-// plain Hessian's row operand is all P planes (halves = P): H = Σ_q XᵀX_q.
-// Each run computes upper tiles only, which is exact for the symmetric sum.
+// (dtype codes 0, 1, 2).
 int dtype_planes(int dtype) { return dtype == 0 ? 1 : dtype == 1 ? 2 : 3; }
-Product x_product(int P) { return Product{false, P}; }
+
+// fp16 activations of a plain Hessian are multiplied as they are: one fp16
+// plane, exact products, one MFMA where the two bf16 planes take four (they
+// remain for GPTAQ's and the weighted operands, whose second factor is not an
+// fp16 value).  C = 4096, 32768 tokens, MI355X: products 2188 -> 609 us, reduces
+// 336 -> 155, staging 236 -> 131; rms distance from fp64 (of
+// sqrt(H_ii·H_jj), C = 4096, 16384 tokens) 3.0e-9 -> 2.8e-9.
+bool native16(int kind, int P) { return kind == 0 && P == 2; }
+
+// A product: Σ over pairs (row plane, column plane) of staged planes, counted
+// from the first plane of each operand.
+struct Product {
+  bool full;                  // all tiles, or the upper triangle of a symmetric sum
+  int planes;                 // the row operand's planes: set the split count (error of a chain)
+  int parts;
+  int a[kMaxParts], b[kMaxParts];
+};
+// X's P planes against themselves, H = Σ X_pᵀX_q (upper tiles of each pair,
+// which is exact for the symmetric sum), smallest pairs first.  An fp32 value
+// is three planes of 8 significant bits: the pairs (1, 2), (2, 1) and (2, 2)
+// are below 2⁻²³ of the product and left out (the others sum to the product
+// of two 24-bit values within fp32's own rounding: rms distance from fp64 at
+// C = 2752, 14000 tokens 4.4e-9 of sqrt(H_ii·H_jj), with all nine pairs
+// 4.7e-9).  All pairs run in one launch: products 1175 -> 714 us, reduces
+// 154 -> 100 (MI355X, that size).
+constexpr Product X1{false, 1, 1, {0}, {0}};
+constexpr Product X2{false, 2, 4, {1, 1, 0, 0}, {1, 0, 1, 0}};
+constexpr Product X3{false, 3, 6, {2, 0, 1, 1, 0, 0}, {0, 2, 1, 0, 1, 0}};
+// The two planes (hi, lo) of a 16-bit operand against X's P planes: GPTAQ's
+// (X_fp − X) and the weighted x·w.  (lo, 2) is below 2⁻²³ and left out.
+constexpr Product V1{false, 2, 2, {0, 1}, {0, 0}};
+constexpr Product V2{false, 2, 4, {1, 0, 1, 0}, {1, 1, 0, 0}};
+constexpr Product V3{false, 2, 5, {0, 1, 0, 1, 0}, {2, 1, 1, 0, 0}};
+Product x_product(int P) { return P == 1 ? X1 : P == 2 ? X2 : X3; }
+Product v_product(int P, bool full) {
+  Product p = P == 1 ? V1 : P == 2 ? V2 : V3;
+  p.full = full;
+  return p;
+}
+Product h_product(int kind, int P) { return native16(kind, P) ? X1 : x_product(P); }
 
 size_t product_ws(int64_t K, int64_t C, Product pr) {
   const int64_t tiles = n_tiles(C, pr.full);
-  return plan_ws_bytes(tiles, gram_plan(tiles, K, pr.halves));
+  return plan_ws_bytes(tiles, gram_plan(tiles, K, pr.planes, pr.parts));
 }
 
 int64_t product_width(int64_t K, int64_t C, Product pr) {
-  return gram_plan(n_tiles(C, pr.full), K, pr.halves).Kp;
+  return gram_plan(n_tiles(C, pr.full), K, pr.planes, pr.parts).Kp;
 }
 
 // The weighted kind of bf16 activations runs all G groups in one
-// wgram_kernel launch over tiles·G work items (no operand halves); with P > 1
-// activation planes it stages the hi/lo planes of x·w and runs SYM2 products.
+// wgram_kernel launch over tiles·G work items (one part); with P > 1
+// activation planes it stages the hi/lo planes of x·w and runs a v_product per group.
 bool fused_weighted(int kind, int P) { return kind == 2 && P == 1; }
 // Each split of a weighted product is also cut to at most kWChain tokens: its
 // fp32 accumulators take two MFMA updates (hi, lo) per 16 tokens, and the
@@ -1033,7 +1077,7 @@ constexpr int64_t kWBudget = int64_t(16) << 30;
 GramPlan wplan(int64_t K, int64_t C, int64_t G) {
   const int64_t items = n_tiles(C, false) * G;
   const int64_t max_s = std::max<int64_t>(1, kWBudget / (items * TT * TT * 4));
-  return gram_plan(items, K, 1, kWChain, max_s);
+  return gram_plan(items, K, 1, 1, kWChain, max_s);
 }
 
 // Feature planes (Cp rows) staged per kind (0 Hessian, 1 GPTAQ, 2 weighted
@@ -1053,16 +1097,19 @@ int64_t kind_height(int kind, int64_t C, int64_t G, int P = 1) {
 
 // Staged token width and Gram workspace a kind needs for K tokens.
 int64_t kind_width(int kind, int64_t K, int64_t C, int P = 1, int64_t G = 1) {
-  if (kind == 0) return product_width(K, C, x_product(P));
-  if (kind == 1) return std::max(product_width(K, C, x_product(P)), product_width(K, C, FULL2));
+  if (kind == 0) return product_width(K, C, h_product(kind, P));
+  if (kind == 1)
+    return std::max(product_width(K, C, h_product(kind, P)),
+                    product_width(K, C, v_product(P, true)));
   if (fused_weighted(kind, P)) return wplan(K, C, G).Kp;
-  return product_width(K, C, SYM2);
+  return product_width(K, C, v_product(P, false));
 }
 size_t kind_gram_ws(int kind, int64_t K, int64_t C, int P = 1, int64_t G = 1) {
-  if (kind == 0) return product_ws(K, C, x_product(P));
-  if (kind == 1) return std::max(product_ws(K, C, x_product(P)), product_ws(K, C, FULL2));
+  if (kind == 0) return product_ws(K, C, h_product(kind, P));
+  if (kind == 1)
+    return std::max(product_ws(K, C, h_product(kind, P)), product_ws(K, C, v_product(P, true)));
   if (fused_weighted(kind, P)) return plan_ws_bytes(n_tiles(C, false) * G, wplan(K, C, G));
-  return product_ws(K, C, SYM2);
+  return product_ws(K, C, v_product(P, false));
 }
 
 // Zero token columns [roundup(K, 64), width) of `rows` staged rows.
@@ -1076,20 +1123,27 @@ int zero_pad(hipStream_t st, uint16_t* XT, int64_t ldt, int64_t rows, int64_t K,
   return G2PTQ_OK;
 }
 
-// out = beta·out + alpha·(product over K staged tokens).  The staged planes
-// must be zero from token roundup(K, 64) up to product_width(K, C, pr).
-int run_product(hipStream_t st, Product pr, const uint16_t* A1, const uint16_t* A2,
-                const uint16_t* A3, const uint16_t* B, int64_t ldt, int64_t K, int64_t C,
-                float alpha, float beta, float* out, int64_t ldo, void* ws, size_t ws_bytes) {
+// out = beta·out + alpha·(product over K staged tokens): pr's pairs of A's and
+// B's planes (`plane` elements apart).  The staged planes must be zero from
+// token roundup(K, 64) up to product_width(K, C, pr).  f16: the planes hold
+// fp16 values.
+int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint16_t* B,
+                int64_t plane, int64_t ldt, int64_t K, int64_t C, float alpha, float beta,
+                float* out, int64_t ldo, void* ws, size_t ws_bytes, bool f16 = false) {
   const int64_t nt = cdiv(C, TT);
   const int64_t tiles = n_tiles(C, pr.full);
-  const GramPlan p = gram_plan(tiles, K, pr.halves);
+  const GramPlan p = gram_plan(tiles, K, pr.planes, pr.parts);
   G2PTQ_CHECK(p.Kp <= ldt, "hessian gram: staged operand too narrow (%lld < %lld)",
               (long long)ldt, (long long)p.Kp);
   G2PTQ_CHECK(tiles * p.S < (1ll << 31) && tiles < 65536, "hessian gram: grid too large");
+  G2PTQ_CHECK(!f16 || !pr.full, "hessian gram: fp16 planes are for symmetric products");
   G2Args a{};
-  a.A1 = A1; a.A2 = A2; a.A3 = A3; a.B = B; a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
-  a.S = p.S; a.halves = pr.halves; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
+  for (int q = 0; q < pr.parts; ++q) {
+    a.A[q] = A + pr.a[q] * plane;
+    a.B[q] = B + pr.b[q] * plane;
+  }
+  a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
+  a.S = p.S; a.parts = pr.parts; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
   a.G = 1;
   if (p.S > 1) {
     const size_t need = plan_ws_bytes(tiles, p);
@@ -1099,7 +1153,10 @@ int run_product(hipStream_t st, Product pr, const uint16_t* A1, const uint16_t* 
   }
   const dim3 grid((unsigned)(tiles * p.S));
   const bool direct_beta = p.S == 1 && beta != 0.f;
-  if (pr.full) {
+  if (f16) {
+    if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, false, true>), grid, dim3(NTH), 0, st, a);
+    else hipLaunchKernelGGL((gram256_kernel<false, false, true>), grid, dim3(NTH), 0, st, a);
+  } else if (pr.full) {
     if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, true>), grid, dim3(NTH), 0, st, a);
     else hipLaunchKernelGGL((gram256_kernel<false, true>), grid, dim3(NTH), 0, st, a);
   } else {
@@ -1133,8 +1190,8 @@ int run_wproduct(hipStream_t st, const uint16_t* XT, const float* W, int64_t ldw
   G2PTQ_CHECK((reinterpret_cast<uintptr_t>(W) & 15) == 0 && ldw % 4 == 0,
               "hessian gram: weights must be 16-byte aligned with ldw a multiple of 4");
   G2Args a{};
-  a.B = XT; a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
-  a.S = p.S; a.halves = 1; a.alpha = alpha; a.beta = beta; a.H = H; a.ldh = ldh;
+  a.B[0] = XT; a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
+  a.S = p.S; a.parts = 1; a.alpha = alpha; a.beta = beta; a.H = H; a.ldh = ldh;
   a.W = W; a.ldw = ldw; a.G = G; a.sH = sH;
   if (p.S > 1) {
     const size_t need = plan_ws_bytes(tiles * G, p);
@@ -1175,13 +1232,12 @@ int stage(hipStream_t st, int kind, const uint16_t* X, const uint16_t* F, const 
   s.t_end = cdiv(T, KS) * KS;
   s.vec = aligned(X, ldx) && (kind != 1 || aligned(F, ldf));
   const dim3 grid((unsigned)cdiv(T, (int64_t)ST_T), (unsigned)(Cp / ST_C));
-  if (dtype == 0) {
+  if (dtype == 0 || native16(kind, dtype_planes(dtype))) {  // 16-bit values as they are
     if (kind == 0) hipLaunchKernelGGL(stage_kernel<0>, grid, dim3(256), 0, st, s);
     else if (kind == 1) hipLaunchKernelGGL(stage_kernel<1>, grid, dim3(256), 0, st, s);
     else hipLaunchKernelGGL(stage_kernel<2>, grid, dim3(256), 0, st, s);
   } else if (dtype == 1) {
-    if (kind == 0) hipLaunchKernelGGL((stage_split_kernel<_Float16, 0>), grid, dim3(256), 0, st, s);
-    else if (kind == 1) hipLaunchKernelGGL((stage_split_kernel<_Float16, 1>), grid, dim3(256), 0, st, s);
+    if (kind == 1) hipLaunchKernelGGL((stage_split_kernel<_Float16, 1>), grid, dim3(256), 0, st, s);
     else hipLaunchKernelGGL((stage_split_kernel<_Float16, 2>), grid, dim3(256), 0, st, s);
   } else {
     if (kind == 0) hipLaunchKernelGGL((stage_split_kernel<float, 0>), grid, dim3(256), 0, st, s);
@@ -1219,31 +1275,23 @@ int gram_kind(hipStream_t st, int kind, uint16_t* XT, int64_t ldt, int64_t K, in
   const int64_t width = kind_width(kind, K, C, P, G);
   G2PTQ_CHECK(width <= ldt, "hessian gram: staged operand too narrow (%lld < %lld)",
               (long long)ldt, (long long)width);
-  G2PTQ_TRY(zero_pad(st, XT, ldt, kind_planes(kind, G, P) * Cp, K, width));
+  G2PTQ_TRY(zero_pad(st, XT, ldt, (native16(kind, P) ? 1 : kind_planes(kind, G, P)) * Cp, K, width));
   if (fused_weighted(kind, P)) {
     // the weight rows, as 2G rows of 2·ldt bf16 elements
     G2PTQ_TRY(zero_pad(st, XT + plane, 2 * ldt, G, 2 * K, 2 * width));
     return run_wproduct(st, XT, reinterpret_cast<const float*>(XT + plane), ldt, ldt, K, C, G,
                         alpha, beta, H, ldh, sH, ws, ws_bytes);
   }
-  const uint16_t* Xq[3] = {XT, XT + plane, XT + 2 * plane};
-  // every product over the column planes q = 0..P−1: the first applies beta,
-  // the others add to it
-  for (int q = 0; q < P; ++q) {
-    const float b = q == 0 ? beta : 1.f;
-    if (kind != 2)
-      G2PTQ_TRY(run_product(st, x_product(P), Xq[0], P > 1 ? Xq[1] : nullptr,
-                            P > 2 ? Xq[2] : nullptr, Xq[q], ldt, K, C, alpha, b, H, ldh, ws,
-                            ws_bytes));
-    if (kind == 1)
-      G2PTQ_TRY(run_product(st, FULL2, XT + P * plane, XT + (P + 1) * plane, nullptr, Xq[q], ldt,
-                            K, C, alpha, b, Dx, ldd, ws, ws_bytes));
-    if (kind == 2)
-      for (int64_t g = 0; g < G; ++g)
-        G2PTQ_TRY(run_product(st, SYM2, XT + (P + 2 * g) * plane, XT + (P + 2 * g + 1) * plane,
-                              nullptr, Xq[q], ldt, K, C, alpha, b, H + g * sH, ldh, ws,
-                              ws_bytes));
-  }
+  if (kind != 2)
+    G2PTQ_TRY(run_product(st, h_product(kind, P), XT, XT, plane, ldt, K, C, alpha, beta, H, ldh, ws,
+                          ws_bytes, native16(kind, P)));
+  if (kind == 1)
+    G2PTQ_TRY(run_product(st, v_product(P, true), XT + P * plane, XT, plane, ldt, K, C, alpha, beta,
+                          Dx, ldd, ws, ws_bytes));
+  if (kind == 2)
+    for (int64_t g = 0; g < G; ++g)
+      G2PTQ_TRY(run_product(st, v_product(P, false), XT + (P + 2 * g) * plane, XT, plane, ldt, K, C,
+                            alpha, beta, H + g * sH, ldh, ws, ws_bytes));
   return G2PTQ_OK;
 }
 

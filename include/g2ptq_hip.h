@@ -183,17 +183,18 @@ int g2ptq_weighted_gram(void* stream, uint16_t* XT, int64_t ldt, int64_t K, int6
  * staged as P bf16 planes that sum to it exactly (P = 1, 2, 3), followed by
  * the kind's planes as above (GPTAQ: hi, lo of X_fp − X; weighted with
  * P > 1: hi, lo of x·S[t,g]·s_scale per group; weighted bf16: the weight
- * rows of g2ptq_weighted_stage); g2ptq_hessian_stage_planes gives the count
- * of feature planes (rows × ldt each) and g2ptq_hessian_stage_height the
- * buffer's height in rows of ldt bf16 (planes × rows, plus the bf16
- * weighted kind's 2G).  g2ptq_hessian_gram_ex runs each product once per plane of Xᵀ as
- * its column operand (the plain Hessian's row operand is all P planes),
- * accumulating: the same H / Dx / H[g] updates as g2ptq_hessian_gram,
- * g2ptq_gptaq_gram and g2ptq_weighted_gram (whose bf16 paths these equal
- * bit for bit), at P times their work for GPTAQ's cross term and the
- * weighted kind and P² times for the plain Hessian.  Same alignment and
- * padding rules as g2ptq_hessian_stage / _gram; act (kind 2) as in
- * g2ptq_weighted_stage. */
+ * rows of g2ptq_weighted_stage); the plain Hessian of fp16 activations stages
+ * them as they are in the first of its two planes and leaves the second
+ * alone.  g2ptq_hessian_stage_planes gives the count of feature planes
+ * (rows × ldt each) and g2ptq_hessian_stage_height the buffer's height in
+ * rows of ldt bf16 (planes × rows, plus the bf16 weighted kind's 2G).
+ * g2ptq_hessian_gram_ex sums each product over the pairs of row and column
+ * planes: one fp16 product for the plain Hessian of fp16, the pairs above
+ * 2⁻²³ of the product for fp32 (6 of 9; 5 of 6 for GPTAQ's cross term and
+ * the weighted kind).  The updates are those of g2ptq_hessian_gram,
+ * g2ptq_gptaq_gram and g2ptq_weighted_gram, whose bf16 paths these equal bit
+ * for bit.  Same alignment and padding rules as g2ptq_hessian_stage / _gram;
+ * act (kind 2) as in g2ptq_weighted_stage. */
 int g2ptq_hessian_stage_planes(int kind, int dtype, int64_t G, int64_t* planes);
 int g2ptq_hessian_stage_height(int kind, int dtype, int64_t C, int64_t G, int64_t* rows);
 int g2ptq_hessian_stage_ex(void* stream, int kind, int dtype, const void* X, const void* Xfp,
