@@ -13,15 +13,16 @@ namespace {
 // workgroup (rows at or past nbk are identity rows), and the inverse
 // X = L⁻¹ by forward substitution, block row by block row:
 //   panel p (wave 0, lane i = row i): the 16 pivots of columns
-//     [16p, 16p + 16) in turn, each d = A[j][j] read from lane j,
-//     l_ij = A[i][j]·rsqrt(d), and the rank-1 update of the panel's own
-//     later columns: the next two with the multipliers of their rows read
-//     from those lanes (v_readlane, on the pivot chain), the rest with the
-//     multipliers the panel rows wrote to LDS (one store and a few
-//     broadcast reads instead of a v_readlane per column; no barrier, the
-//     wave's LDS accesses complete in order);
-//   trailing update (all waves): A[i][c] −= Σ_t l_it·l_ct over the panel's
-//     16 columns for 16p + 16 <= c <= i, 4×2 or 2×2 entries per thread;
+//     [16p, 16p + 16) in turn, each d = A[j][j], l_ij = A[i][j]·rsqrt(d), and
+//     the rank-1 update of the panel's own later columns.  Every 16-lane DPP
+//     row also carries the panel's 16×16 diagonal block (lane i: its row
+//     i % 16), so that pivots and multipliers reach all lanes by DPP row
+//     broadcasts inside the row: no LDS round trip and no v_readlane on the
+//     pivot chain, for 16 more fused multiply-adds per lane and pivot at most;
+//   trailing update (waves 0 to 2): A[i][c] −= Σ_t l_it·l_ct over the panel's
+//     16 columns for 16p + 16 <= c <= i, by 16×16 tiles on
+//     v_mfma_f32_16x16x4_f32, which is the ascending chain of four fused
+//     multiply-adds per entry bit for bit (measured on MI355X);
 //   inverse rows [16p, 16p + 16) (one of waves 1 to 3, lane i = column i,
 //     beside the later panels): acc_r = δ_ri − Σ_{j<r} X[j][i]·l_rj,
 //     X[r][i] = acc_r·rsqrt(d_r).
@@ -37,205 +38,211 @@ constexpr int POT_NB = 64;          // block edge
 constexpr int XP = POT_NB + 1;      // LDS row pitch of the block / X buffer
 constexpr int LP = POT_NB + 4;      // LDS row pitch of L (16-byte rows)
 constexpr int PB = 16;              // panel width
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float lane_val(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+// Lane O of each 16-lane row to the whole row (DPP row_newbcast:O).
+template <int O>
+__device__ __forceinline__ float row_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + O, 0xf, 0xf, true));
 }
 
-// Panel P's 16 pivot steps on wave 0: rows from As, L columns to Lm, 1/sqrt
-// of the pivots to rdv.  The multipliers and pivots stay in registers until
-// the panel is done (Lm gets whole 16-byte rows, zeros on and above the
-// diagonal, which nothing reads), so the pivot chain carries no stores.
-template <int P>
-__device__ __forceinline__ void pot_panel(const float* As, float* Lm, float* rdv, int i, int& fail) {
-  constexpr int k0 = P * PB;
-  constexpr int LA = 2;  // columns after the pivot updated through v_readlane
-  float* Mb = rdv + POT_NB;  // per pivot, the panel rows' multipliers (LDS)
-  float a[PB], l[PB];
-  float rdl = 0.f;  // lane j: 1/sqrt of pivot k0 + j
+// c −= bcast(mp, lane C of each row)·m, one fused multiply-add with the
+// broadcast on its operand (the compiler keeps a separate v_mov_b32_dpp).  A
+// DPP operand needs two wait states after the VALU write of its register:
+// FIRST carries them for a pivot's mp and orders the other uses behind it
+// (the compiler sees no hazard inside inline assembly; operands that come from
+// LDS need none).
+template <int C, bool FIRST>
+__device__ __forceinline__ void row_fma(float& c, float& mp, float m) {
+  if constexpr (FIRST)
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(c), "+v"(mp) : "v"(m), "n"(C));
+  else
+    asm("v_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+        : "+v"(c) : "v"(mp), "v"(m), "n"(C));
+}
+
+// The panel's columns C, C + 1, … after pivot J with multipliers m (the
+// lane's row) and mp (the diagonal block's row).
+template <int J, int C>
+__device__ __forceinline__ void pot_update(float (&a)[PB], float (&p)[PB], float m, float& mp) {
+  if constexpr (C < PB) {
+    row_fma<C, C == J + 1>(p[C], mp, mp);
+    row_fma<C, false>(a[C], mp, m);
+    pot_update<J, C + 1>(a, p, m, mp);
+  }
+}
+
+// A panel's pivot J and the ones after it: lane i holds row i's panel columns
+// in a, and row k0 + i % 16's (of the panel's diagonal block) in p.
+template <int J>
+__device__ __forceinline__ void pot_pivots(float (&a)[PB], float (&p)[PB], float (&l)[PB],
+                                           float& rdl, float& dl, int i) {
+  if constexpr (J < PB) {
+    const float d = row_lane<J>(p[J]);
+    const float rd = __builtin_amdgcn_rsqf(d);
+    float mp = p[J] * rd;
+    const float m = a[J] * rd;
+    l[J] = m;
+    rdl = (i == J) ? rd : rdl;
+    dl = (i == J) ? d : dl;
+    pot_update<J, J + 1>(a, p, m, mp);
+    pot_pivots<J + 1>(a, p, l, rdl, dl, i);
+  }
+}
+
+// The 16 pivot steps of the panel at column k0 on wave 0: rows from As, L
+// columns to Lm, 1/sqrt of the pivots to rdv.  (Rows above a pivot carry values that nothing reads:
+// Lm is read below the diagonal only.)
+__device__ __forceinline__ void pot_panel(const float* As, float* Lm, float* rdv, int k0, int i,
+                                          int& fail) {
+  float a[PB], p[PB], l[PB];
+  float rdl = 0.f, dl = 1.f;  // lane j: 1/sqrt of pivot k0 + j, and the pivot
+#pragma unroll
+  for (int c = 0; c < PB; ++c) p[c] = As[(k0 + (i & 15)) * XP + k0 + c];
 #pragma unroll
   for (int c = 0; c < PB; ++c) a[c] = As[i * XP + k0 + c];
-#pragma unroll
-  for (int j = 0; j < PB; ++j) {
-    const float d = lane_val(a[j], k0 + j);
-    fail = (fail == 0 && !(d > 0.f)) ? k0 + j + 1 : fail;  // also catches NaN
-    const float rd = __builtin_amdgcn_rsqf(d);
-    const float m = (i > k0 + j) ? a[j] * rd : 0.f;
-    l[j] = m;
-    rdl = (i == j) ? rd : rdl;
-    if (j + LA + 1 < PB && i >= k0 && i < k0 + PB) Mb[j * PB + (i - k0)] = m;
-#pragma unroll
-    for (int c = j + 1; c < PB && c <= j + LA; ++c)
-      a[c] = __builtin_fmaf(-m, lane_val(m, k0 + c), a[c]);
-#pragma unroll
-    for (int c = j + LA + 1; c < PB; ++c) a[c] = __builtin_fmaf(-m, Mb[j * PB + c], a[c]);
-  }
+  pot_pivots<0>(a, p, l, rdl, dl, i);
 #pragma unroll
   for (int c4 = 0; c4 < PB; c4 += 4)
     *reinterpret_cast<float4*>(&Lm[i * LP + k0 + c4]) = make_float4(l[c4], l[c4 + 1], l[c4 + 2], l[c4 + 3]);
   if (i < PB) rdv[k0 + i] = rdl;
+  const uint64_t bad = __builtin_amdgcn_ballot_w64(!(dl > 0.f));  // also catches NaN
+  if (fail == 0 && bad) fail = k0 + __builtin_ctzll(bad) + 1;
 }
 
-// Trailing update by panel P of the lower entries at or past column 16P + 16,
-// in blocks of RB rows × 2 columns on or below the diagonal, one per thread:
-// 4-row blocks where 2×2 blocks would not fit in one pass of the 256 threads
-// (panel 0: 156 blocks of 4×2 instead of 300 of 2×2), 2×2 otherwise.
-template <int P>
-__device__ __forceinline__ void pot_trail(float* As, const float* Lm) {
-  constexpr int k0 = P * PB, t0 = k0 + PB, W = POT_NB - t0;
-  constexpr int RB = (W / 2) * (W / 2 + 1) / 2 > 256 ? 4 : 2;
-  constexpr int NR = W / RB;  // row blocks; row block ib has RB / 2·ib + RB / 2 column pairs
-  constexpr int NLOW = RB == 4 ? NR * (NR + 1) : NR * (NR + 1) / 2;
-  static_assert(NLOW <= 256, "one pass");
-  const int q = threadIdx.x;
-  if (q >= NLOW) return;
-  // blocks before row block ib: ib·(ib + 1) (RB = 4) or ib·(ib + 1)/2 (RB = 2)
-  const float qf = RB == 4 ? (float)q : 2.f * (float)q;
-  int ib = (int)((sqrtf(4.f * qf + 1.f) - 1.f) * 0.5f);
-  auto before = [](int v) { return RB == 4 ? v * (v + 1) : v * (v + 1) / 2; };
-  while (before(ib) > q) --ib;
-  while (before(ib + 1) <= q) ++ib;
-  const int cb = q - before(ib);
-  const int r0 = t0 + RB * ib, c0 = t0 + 2 * cb;
-  float acc[RB][2];
+// Trailing update by the panel at column k0 of the lower entries at or past
+// column k0 + 16: the 16×16 tiles on or below the diagonal, dealt to waves 0
+// to 2 (6, 3 and 1 tiles).  Four K = 4 MFMAs per tile in increasing column
+// order; a lane holds rows 4·(lane / 16) + v and column lane % 16 of a tile.
+__device__ __forceinline__ void pot_trail(float* As, const float* Lm, int k0, int i, int w) {
+  const int t0 = k0 + PB, nt = (POT_NB - t0) / 16;
+  const int r16 = i & 15, g = i >> 4;
+#pragma unroll 1
+  for (int q = w; q < nt * (nt + 1) / 2; q += 3) {
+    const int ti = q >= 3 ? 2 : q >= 1 ? 1 : 0, tj = q - ti * (ti + 1) / 2;
+    const int r0 = t0 + 16 * ti, c0 = t0 + 16 * tj;
+    float av[4], bv[4];
 #pragma unroll
-  for (int r = 0; r < RB; ++r)
+    for (int s = 0; s < 4; ++s) {
+      av[s] = -Lm[(r0 + r16) * LP + k0 + 4 * s + g];
+      bv[s] = Lm[(c0 + r16) * LP + k0 + 4 * s + g];
+    }
+    f32x4 acc;
 #pragma unroll
-    for (int c = 0; c < 2; ++c) acc[r][c] = As[(r0 + r) * XP + c0 + c];
+    for (int v = 0; v < 4; ++v) acc[v] = As[(r0 + 4 * g + v) * XP + c0 + r16];
 #pragma unroll
-  for (int t4 = 0; t4 < PB; t4 += 4) {
-    float4 li[RB], lc[2];
+    for (int s = 0; s < 4; ++s)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < RB; ++r) li[r] = *reinterpret_cast<const float4*>(&Lm[(r0 + r) * LP + k0 + t4]);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) lc[c] = *reinterpret_cast<const float4*>(&Lm[(c0 + c) * LP + k0 + t4]);
-#pragma unroll
-    for (int r = 0; r < RB; ++r)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        acc[r][c] = __builtin_fmaf(-li[r].x, lc[c].x, acc[r][c]);
-        acc[r][c] = __builtin_fmaf(-li[r].y, lc[c].y, acc[r][c]);
-        acc[r][c] = __builtin_fmaf(-li[r].z, lc[c].z, acc[r][c]);
-        acc[r][c] = __builtin_fmaf(-li[r].w, lc[c].w, acc[r][c]);
-      }
+    for (int v = 0; v < 4; ++v)
+      As[(r0 + 4 * g + v) * XP + c0 + r16] = acc[v];  // above the diagonal: not read
   }
-#pragma unroll
-  for (int r = 0; r < RB; ++r)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      if (c0 + c <= r0 + r) As[(r0 + r) * XP + c0 + c] = acc[r][c];
 }
 
-// Rows [16P, 16P + 16) of X = L⁻¹, lane i = column i (one wave), in three
-// parts so that the bulk of the later block rows runs beside the panels:
-//   pot_inv_init: acc_q = δ(16P + q, i);
-//   pot_inv_bulk: acc_q −= Σ_{jlo <= j < jhi} X[j][i]·l_{16P+q, j}, j in
-//     increasing order (X rows below jhi final in Xs);
+// Rows [r0, r0 + 16) of X = L⁻¹, lane i = column i (one wave), in three parts
+// so that the bulk of the later block rows runs beside the panels:
+//   acc_q = δ(r0 + q, i) to begin with;
+//   pot_inv_bulk: acc_q −= Σ_{j0 <= j < j0 + 16} X[j][i]·l_{r0+q, j}, j in
+//     increasing order (X rows below j0 + 16 final in Xs);
 //   pot_inv_fin:  the block's own triangle and the rows into Xs.
 // Each entry receives the same fused multiply-adds in the same order however
-// the j range is split, so the split is invisible in the results.
-template <int P>
-__device__ __forceinline__ void pot_inv_init(float (&acc)[PB], int i) {
-  constexpr int r0 = P * PB;
+// the j range is split, so the split is invisible in the results.  Lane i
+// holds L's row r0 + i % 16, so that l_{r0+q, j} reaches the lanes as a row
+// broadcast: 16 LDS words per lane and 16 columns instead of one broadcast
+// read per multiplier.
+// Sixteen columns from j0 of L's row r0 + i % 16.
+__device__ __forceinline__ void pot_load_l(float (&l)[PB], const float* Lm, int r0, int j0, int i) {
 #pragma unroll
-  for (int q = 0; q < PB; ++q) acc[q] = (r0 + q == i) ? 1.f : 0.f;
+  for (int u = 0; u < PB; u += 4) {
+    const float4 v = *reinterpret_cast<const float4*>(&Lm[(r0 + (i & 15)) * LP + j0 + u]);
+    l[u] = v.x; l[u + 1] = v.y; l[u + 2] = v.z; l[u + 3] = v.w;
+  }
 }
 
-template <int P, int JLO, int JHI>
+// acc[q] −= l_q·x for q >= Q, l_q on lane q of each row.
+template <int Q>
+__device__ __forceinline__ void pot_axpy(float (&acc)[PB], float& l, float x) {
+  if constexpr (Q < PB) {
+    row_fma<Q, false>(acc[Q], l, x);
+    pot_axpy<Q + 1>(acc, l, x);
+  }
+}
+
 __device__ __forceinline__ void pot_inv_bulk(float (&acc)[PB], const float* Xs, const float* Lm,
+                                             int r0, int j0, int i) {
+  float l[PB], x[PB];
+  pot_load_l(l, Lm, r0, j0, i);
+#pragma unroll
+  for (int j = 0; j < PB; ++j) x[j] = Xs[(j0 + j) * XP + i];
+#pragma unroll
+  for (int j = 0; j < PB; ++j) pot_axpy<0>(acc, l[j], x[j]);
+}
+
+template <int Q>
+__device__ __forceinline__ void pot_inv_rows(float (&acc)[PB], float (&l)[PB], float rd, float* X,
                                              int i) {
-  constexpr int r0 = P * PB;
-  static_assert(JHI <= r0 && JLO % 4 == 0 && JHI % 4 == 0, "bulk columns left of the block");
-#pragma unroll 1
-  for (int j4 = JLO; j4 < JHI; j4 += 4) {
-    float x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = Xs[(j4 + u) * XP + i];
-#pragma unroll
-    for (int q = 0; q < PB; ++q) {
-      const float4 l = *reinterpret_cast<const float4*>(&Lm[(r0 + q) * LP + j4]);
-      acc[q] = __builtin_fmaf(-x[0], l.x, acc[q]);
-      acc[q] = __builtin_fmaf(-x[1], l.y, acc[q]);
-      acc[q] = __builtin_fmaf(-x[2], l.z, acc[q]);
-      acc[q] = __builtin_fmaf(-x[3], l.w, acc[q]);
-    }
+  if constexpr (Q < PB) {
+    const float x = acc[Q] * row_lane<Q>(rd);
+    X[Q * XP + i] = x;
+    pot_axpy<Q + 1>(acc, l[Q], x);
+    pot_inv_rows<Q + 1>(acc, l, rd, X, i);
   }
 }
 
-template <int P>
 __device__ __forceinline__ void pot_inv_fin(float (&acc)[PB], float* Xs, const float* Lm,
-                                            const float* rdv, int i) {
-  constexpr int r0 = P * PB;
-#pragma unroll
-  for (int q = 0; q < PB; ++q) {
-    const float x = acc[q] * rdv[r0 + q];
-    Xs[(r0 + q) * XP + i] = x;
-#pragma unroll
-    for (int q2 = q + 1; q2 < PB; ++q2)
-      acc[q2] = __builtin_fmaf(-x, Lm[(r0 + q2) * LP + r0 + q], acc[q2]);
-  }
+                                            const float* rdv, int r0, int i) {
+  float l[PB];
+  pot_load_l(l, Lm, r0, r0, i);
+  pot_inv_rows<0>(acc, l, rdv[r0 + (i & 15)], Xs + r0 * XP, i);
 }
 
 // The factor of the block staged in Xs (lower triangle, identity padded),
-// by a 256-thread workgroup.  Lm (64·LP floats) and rdv (64 + 16·16) are scratch.
+// by a 256-thread workgroup.  Lm (64·LP floats) and rdv (64) are scratch.
 // Leaves X = L⁻¹ in Xs (rows, lower triangle; what lies above is not
 // defined) and returns the failing pivot index + 1, or 0.
-// Schedule (waves w0..w3, `|` a barrier; the trailing updates occupy the
-// first 156, 136 and 36 threads):
-//   panel0 | trail0, inv0 (w3) |
+// Schedule (waves w0..w3, `|` a barrier; the trailing updates' tiles on w0 to
+// w2, block rows of the inverse on w3, w3, w1 and w2):
+//   panel0 | trail0, inv0 triangle (w3) |
 //   panel1, inv2[j < 16] (w1), inv3[j < 16] (w2), inv1[j < 16] (w3) |
 //   trail1, inv1 triangle (w3) |
 //   panel2, inv2[16 <= j < 32] (w1), inv3[16 <= j < 32] (w2) |
 //   trail2, inv2 triangle (w1) | panel3, inv3[32 <= j < 48] (w2) | inv3 triangle (w2)
-// so only the last block row's triangle follows the last panel.
+// so only the last block row's triangle follows the last panel.  The four
+// rounds are a loop: a workgroup runs this code once, so a straight-line
+// schedule (62 KB in potrf_diag_kernel) waits for its instructions.
+// MI355X, one workgroup alone: 15.9 thousand cycles (21.2 with v_readlane
+// and LDS multipliers, VALU trailing updates and the straight-line schedule),
+// of which the pivots 2,400 per panel: a fused multiply-add with a DPP operand
+// issues in eight cycles, so a panel's 240 are 1,920 of them.
 __device__ __forceinline__ int potrf_core(float* Xs, float* Lm, float* rdv, int* fail_s) {
-  const int i = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int fail = 0;
-  float acc[PB];  // the wave's inverse block row (waves 1 to 3)
-  if (w == 0) pot_panel<0>(Xs, Lm, rdv, i, fail);
-  __syncthreads();
-  pot_trail<0>(Xs, Lm);
-  if (w == 3) {
-    pot_inv_init<0>(acc, i);
-    pot_inv_fin<0>(acc, Xs, Lm, rdv, i);
+  int own = w == 1 ? 2 : w == 2 ? 3 : 0;  // the wave's block row of the inverse
+  float acc[PB];
+#pragma unroll
+  for (int q = 0; q < PB; ++q) acc[q] = (own * PB + q == i) ? 1.f : 0.f;
+#pragma unroll 1
+  for (int p = 0; p < 4; ++p) {
+    if (w == 0) {
+      pot_panel(Xs, Lm, rdv, p * PB, i, fail);
+    } else if (p > 0 && p <= own) {
+      pot_inv_bulk(acc, Xs, Lm, own * PB, (p - 1) * PB, i);
+    }
+    __syncthreads();
+    if (w < 3) pot_trail(Xs, Lm, p * PB, i, w);
+    if (w != 0 && own == p) {
+      pot_inv_fin(acc, Xs, Lm, rdv, p * PB, i);
+      if (p == 0) {  // w3 goes on with block row 1
+        own = 1;
+#pragma unroll
+        for (int q = 0; q < PB; ++q) acc[q] = (PB + q == i) ? 1.f : 0.f;
+      }
+    }
+    if (p == 3 && threadIdx.x == 0) *fail_s = fail;
+    __syncthreads();
   }
-  __syncthreads();
-  if (w == 0) {
-    pot_panel<1>(Xs, Lm, rdv, i, fail);
-  } else if (w == 1) {
-    pot_inv_init<2>(acc, i);
-    pot_inv_bulk<2, 0, 16>(acc, Xs, Lm, i);
-  } else if (w == 2) {
-    pot_inv_init<3>(acc, i);
-    pot_inv_bulk<3, 0, 16>(acc, Xs, Lm, i);
-  } else {
-    pot_inv_init<1>(acc, i);
-    pot_inv_bulk<1, 0, 16>(acc, Xs, Lm, i);
-  }
-  __syncthreads();
-  pot_trail<1>(Xs, Lm);
-  if (w == 3) pot_inv_fin<1>(acc, Xs, Lm, rdv, i);
-  __syncthreads();
-  if (w == 0) {
-    pot_panel<2>(Xs, Lm, rdv, i, fail);
-  } else if (w == 1) {
-    pot_inv_bulk<2, 16, 32>(acc, Xs, Lm, i);
-  } else if (w == 2) {
-    pot_inv_bulk<3, 16, 32>(acc, Xs, Lm, i);
-  }
-  __syncthreads();
-  pot_trail<2>(Xs, Lm);
-  if (w == 1) pot_inv_fin<2>(acc, Xs, Lm, rdv, i);
-  __syncthreads();
-  if (w == 0) {
-    pot_panel<3>(Xs, Lm, rdv, i, fail);
-  } else if (w == 2) {
-    pot_inv_bulk<3, 32, 48>(acc, Xs, Lm, i);
-  }
-  __syncthreads();
-  if (w == 2) pot_inv_fin<3>(acc, Xs, Lm, rdv, i);
-  if (threadIdx.x == 0) *fail_s = fail;
-  __syncthreads();
   return *fail_s;
 }
 
