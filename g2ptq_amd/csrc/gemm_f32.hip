@@ -81,6 +81,11 @@ __device__ __forceinline__ void split3(float4 u0, float4 u1, bf16x8& h, bf16x8& 
                               __builtin_shufflevector(l2, l3, 0, 1, 2, 3), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// v, or zeros where it is not to be kept.
+__device__ __forceinline__ float4 keep4(float4 v, bool keep) {
+  return make_float4(keep ? v.x : 0.f, keep ? v.y : 0.f, keep ? v.z : 0.f, keep ? v.w : 0.f);
+}
+
 constexpr int BK = 32;
 constexpr int PK = 36;   // [row][k] pitch (floats)
 // Split path: 16-k slabs, each operand staged in LDS as three bf16 planes
@@ -102,6 +107,71 @@ __device__ __forceinline__ void tile_of(int64_t id, int64_t tm, int64_t tn, int6
   in = r / h;
 }
 
+// The tile of this workgroup of a tm × tn grid (tri: GemmF32's).
+__device__ __forceinline__ void gemm_tile(int tri, int64_t tm, int64_t tn, int64_t& im,
+                                          int64_t& in) {
+  const int64_t nwg = gridDim.x, bid = blockIdx.x;
+  if (tri == 0) {
+    // XCD-aware renumbering (workgroups go round-robin over 8 XCDs): every
+    // XCD gets a contiguous range of the grouped tile order.
+    const int64_t q8 = nwg >> 3, r8 = nwg & 7, xcd = bid & 7;
+    const int64_t id = xcd * q8 + (xcd < r8 ? xcd : r8) + (bid >> 3);
+    tile_of(id, tm, tn, im, in);
+  } else if (tri & 8) {
+    // Triangular upper B: tile (im, in) multiplies at most n0 + BN columns
+    // (fewer still when A is upper too), so the work grows to the right.
+    // Longest first: bands of GH tile-columns from the right, each walked
+    // row by row from the top, in dispatch order.
+    const int64_t per = GH * tm;
+    const int64_t band = bid / per, r = bid - band * per;
+    const int64_t c0 = band * GH;
+    const int64_t h = tn - c0 < GH ? tn - c0 : GH;
+    in = tn - 1 - (c0 + r % h);
+    im = r / h;
+  } else if (tri & 2) {
+    // Triangular B: tile (im, in) multiplies K − n0 columns, so the work falls
+    // from left to right.  Longest first: bands of GH tile-columns from the
+    // left, each walked row by row, in dispatch order (no renumbering, so the
+    // 8 XCDs share every band evenly; consecutive tiles of a row land on
+    // different XCDs, each XCD keeping to one column of the band).
+    const int64_t per = GH * tm;
+    const int64_t band = bid / per, r = bid - band * per;
+    const int64_t c0 = band * GH;
+    const int64_t h = tn - c0 < GH ? tn - c0 : GH;
+    in = c0 + r % h;
+    im = r / h;
+  } else {
+    // Triangular A: tile (im, in) multiplies m0 + BM columns, so the work
+    // grows downwards.  Longest first: the grouped order from the bottom
+    // group up, in dispatch order (each XCD keeps to one row of a group).
+    tile_of(bid, tm, tn, im, in);
+    im = tm - 1 - im;
+  }
+}
+
+template <bool B>
+struct BoolTag {
+  static constexpr bool value = B;
+};
+
+// Byte offset from row r0 of an operand's row r0 + r (the last of its R rows
+// where that is past it) and column c: below 2³² for r < 256 and ld < 2²²
+// (gemm_f32's VEC).
+__device__ __forceinline__ uint32_t row_offset(int64_t r0, int r, int64_t R, int64_t ld, int c) {
+  const int64_t last = R - 1 - r0;
+  return (uint32_t)(((r < last ? r : last) * ld + c) * 4);
+}
+
+// K range of the tile at (m0, n0): triangular operands contribute nothing
+// outside it.
+__device__ __forceinline__ void gemm_krange(int tri, int64_t m0, int64_t n0, int64_t bm, int64_t bn,
+                                            int64_t& klo, int64_t& K) {
+  if (tri & 1) K = K < m0 + bm ? K : m0 + bm;
+  if (tri & 2) klo = n0 / BK * BK;
+  if ((tri & 4) && m0 / BK * BK > klo) klo = m0 / BK * BK;
+  if (tri & 8) K = K < n0 + bn ? K : n0 + bn;
+}
+
 // TILE × TILE output per workgroup (4 waves in 2×2, each TILE/2 square made
 // of 32×32 MFMA blocks): 128 for large products, 64 when a 128 grid would
 // leave most CUs idle (the factor's TRSM / panel updates, short tails).
@@ -121,44 +191,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   const int z = blockIdx.z;
   const int64_t b1 = z / g.batch2, b2 = z % g.batch2;
   if (g.skip && g.skip[b1]) return;
-  const int64_t nwg = gridDim.x, bid = blockIdx.x;
   int64_t im, in;
-  if (g.tri == 0) {
-    // XCD-aware renumbering (workgroups go round-robin over 8 XCDs): every
-    // XCD gets a contiguous range of the grouped tile order.
-    const int64_t q8 = nwg >> 3, r8 = nwg & 7, xcd = bid & 7;
-    const int64_t id = xcd * q8 + (xcd < r8 ? xcd : r8) + (bid >> 3);
-    tile_of(id, tm, tn, im, in);
-  } else if (g.tri & 8) {
-    // Triangular upper B: tile (im, in) multiplies at most n0 + BN columns
-    // (fewer still when A is upper too), so the work grows to the right.
-    // Longest first: bands of GH tile-columns from the right, each walked
-    // row by row from the top, in dispatch order.
-    const int64_t per = GH * tm;
-    const int64_t band = bid / per, r = bid - band * per;
-    const int64_t c0 = band * GH;
-    const int64_t h = tn - c0 < GH ? tn - c0 : GH;
-    in = tn - 1 - (c0 + r % h);
-    im = r / h;
-  } else if (g.tri & 2) {
-    // Triangular B: tile (im, in) multiplies K − n0 columns, so the work falls
-    // from left to right.  Longest first: bands of GH tile-columns from the
-    // left, each walked row by row, in dispatch order (no renumbering, so the
-    // 8 XCDs share every band evenly; consecutive tiles of a row land on
-    // different XCDs, each XCD keeping to one column of the band).
-    const int64_t per = GH * tm;
-    const int64_t band = bid / per, r = bid - band * per;
-    const int64_t c0 = band * GH;
-    const int64_t h = tn - c0 < GH ? tn - c0 : GH;
-    in = c0 + r % h;
-    im = r / h;
-  } else {
-    // Triangular A: tile (im, in) multiplies m0 + BM columns, so the work
-    // grows downwards.  Longest first: the grouped order from the bottom
-    // group up, in dispatch order (each XCD keeps to one row of a group).
-    tile_of(bid, tm, tn, im, in);
-    im = tm - 1 - im;
-  }
+  gemm_tile(g.tri, tm, tn, im, in);
   const int64_t m0 = im * BM, n0 = in * BN;
   if (g.uplo == 1 && n0 > m0 + BM - 1) return;
   if (g.uplo == 2 && m0 > n0 + BN - 1) return;
@@ -166,12 +200,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   const float* __restrict__ A = g.A + b1 * g.sA + b2 * g.sA2;
   const float* __restrict__ B = g.B + b1 * g.sB + b2 * g.sB2;
   const int64_t M = g.M, N = g.N;
-  // K range of this tile: triangular operands contribute nothing outside it.
   int64_t klo = 0, K = g.K;
-  if (g.tri & 1) K = K < m0 + BM ? K : m0 + BM;
-  if (g.tri & 2) klo = n0 / BK * BK;
-  if ((g.tri & 4) && m0 / BK * BK > klo) klo = m0 / BK * BK;
-  if (g.tri & 8) K = K < n0 + BN ? K : n0 + BN;
+  gemm_krange(g.tri, m0, n0, BM, BN, klo, K);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -183,16 +213,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   const int ra_row = tid >> 3, ra_kq = (tid & 7) * 4;
   const int rb_k = tid / KQ, rb_nq = (tid % KQ) * 4;
 
+  // Loads are issued raw from clamped addresses and masked where they are
+  // stored to LDS, one to four slabs later: a mask at the load makes the wave
+  // wait for memory in the very slab that issues it.  Only k needs a mask:
+  // rows (columns) past M (N) are multiplied and never stored.  With VEC a
+  // 16-byte chunk is wholly inside or outside the k range.  MI355X, masks at
+  // the loads before, split products: 512×2048×2048 (64×64 tiles) 61 -> 47 us,
+  // 512×8192×8192 (128×128) 522 -> 404, 1024×4096×4096 four times (256×256)
+  // 682 -> 644.
   auto ld4 = [&](const float* base, int64_t ld, int64_t r, int64_t c, int64_t R, int64_t Ccols) {
     if (VEC) {
-      // Rows of a multiple of 4 columns (c is one): a 16-byte chunk is wholly
-      // inside or outside, so one load from a clamped address and a select
-      // replace per-element tests (no branches).
-      const bool ok = r < R && c < Ccols;
-      const uint4 w = *reinterpret_cast<const uint4*>(base + (ok ? r * ld + c : 0));
-      const uint32_t m = ok ? 0xffffffffu : 0u;  // a mask, not a branch around the load
-      return make_float4(__uint_as_float(w.x & m), __uint_as_float(w.y & m),
-                         __uint_as_float(w.z & m), __uint_as_float(w.w & m));
+      return *reinterpret_cast<const float4*>(base + (r < R ? r : R - 1) * ld + (c < Ccols ? c : 0));
     }
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (r < R) {
@@ -217,15 +248,20 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
       else RBr[i_] = ld4(B, g.ldb, k0_ + rb_k + RB_ROWS * i_, n0 + rb_nq, K, N);                \
     }                                                                                          \
   } while (0)
-#define GF_STORE(RAr, RBr, buf)                                                                \
+#define GF_STORE(RAr, RBr, buf, slab)                                                          \
   do {                                                                                         \
+    const int64_t k0_ = klo + (int64_t)(slab) * BK;                                            \
+    const bool ka_ = k0_ + ra_kq < K;                                                          \
     _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                          \
-      *reinterpret_cast<float4*>(&As[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) = RAr[i_];       \
+      *reinterpret_cast<float4*>(&As[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) =                \
+          keep4(RAr[i_], ka_);                                                                 \
     _Pragma("unroll") for (int i_ = 0; i_ < RB; ++i_) {                                        \
       if (B_KCONTIG)                                                                           \
-        *reinterpret_cast<float4*>(&Bs[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) = RBr[i_];     \
+        *reinterpret_cast<float4*>(&Bs[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) =              \
+            keep4(RBr[i_], ka_);                                                               \
       else                                                                                     \
-        *reinterpret_cast<float4*>(&Bs[(buf)][(rb_k + RB_ROWS * i_) * PN + rb_nq]) = RBr[i_];  \
+        *reinterpret_cast<float4*>(&Bs[(buf)][(rb_k + RB_ROWS * i_) * PN + rb_nq]) =           \
+            keep4(RBr[i_], k0_ + rb_k + RB_ROWS * i_ < K);                                     \
     }                                                                                          \
   } while (0)
 
@@ -314,59 +350,52 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
     __bf16* const Ap = reinterpret_cast<__bf16*>(&As[0][0]);  // [buf][plane][row][SP]
     __bf16* const Bp = reinterpret_cast<__bf16*>(&Bs[0][0]);
     constexpr int RS = TILE / 64;                          // float4 per thread ([row][k])
-    constexpr int KPT = SK * TILE / 256;                   // B as K×N: k per thread (8 or 4)
     const int sa_row = tid >> 2, sa_kq = (tid & 3) * 4;
-    const int sb_n = tid % TILE, sb_k = (tid / TILE) * KPT;
-    const uint32_t b_off = B_KCONTIG ? 0u : (uint32_t)(sb_k * g.ldb + sb_n);
+    const int nk = K > klo ? (int)cdiv(K - klo, (int64_t)SK) : 0;
     float4 ra0[RS], ra1[RS], ra2[RS], ra3[RS];
     float4 rb0[RS], rb1[RS], rb2[RS], rb3[RS];
-    float bs0[KPT], bs1[KPT], bs2[KPT], bs3[KPT];
-#define GS_LOAD(RA_, RB_, BS_, slab)                                                           \
+    // INNER (a whole number of 16-k slabs, 16-byte loads): no masks, and a
+    // slab's address is a uniform base plus a 32-bit offset per thread (slabs
+    // past the end re-read the last one and go unused).
+    uint32_t oa[RS], ob[RS];
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+      oa[i] = row_offset(m0, sa_row + 64 * i, M, g.lda, sa_kq);
+      ob[i] = row_offset(n0, sa_row + 64 * i, N, g.ldb, sa_kq);
+    }
+    const char* const ua = reinterpret_cast<const char*>(A + m0 * g.lda + klo);
+    const char* const ub = reinterpret_cast<const char*>(B + n0 * g.ldb + klo);
+#define GS_LOAD(RA_, RB_, slab)                                                                \
   do {                                                                                         \
-    const int64_t k0_ = klo + (int64_t)(slab) * SK;                                            \
-    _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_)                                          \
-      RA_[i_] = ld4(A, g.lda, m0 + sa_row + 64 * i_, k0_ + sa_kq, M, K);                       \
-    if (B_KCONTIG) {                                                                           \
-      _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_)                                        \
-        RB_[i_] = ld4(B, g.ldb, n0 + sa_row + 64 * i_, k0_ + sa_kq, N, K);                     \
+    if constexpr (INNER) {                                                                     \
+      const int64_t sl_ = (int64_t)((slab) < nk ? (slab) : nk - 1) * (SK * 4);                 \
+      _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_) {                                      \
+        RA_[i_] = *reinterpret_cast<const float4*>(ua + sl_ + oa[i_]);                         \
+        RB_[i_] = *reinterpret_cast<const float4*>(ub + sl_ + ob[i_]);                         \
+      }                                                                                        \
     } else {                                                                                   \
-      /* uniform row base + a 32-bit per-thread offset */                                      \
-      const bool n_ok_ = n0 + sb_n < N;                                                        \
-      _Pragma("unroll") for (int c_ = 0; c_ < KPT; ++c_) {                                     \
-        const float* row_ = B + (k0_ + c_) * g.ldb + n0;                                       \
-        BS_[c_] = (n_ok_ && k0_ + sb_k + c_ < K) ? row_[b_off] : 0.f;                          \
+      const int64_t k0_ = klo + (int64_t)(slab) * SK;                                          \
+      _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_) {                                      \
+        RA_[i_] = ld4(A, g.lda, m0 + sa_row + 64 * i_, k0_ + sa_kq, M, K);                     \
+        RB_[i_] = ld4(B, g.ldb, n0 + sa_row + 64 * i_, k0_ + sa_kq, N, K);                     \
       }                                                                                        \
     }                                                                                          \
   } while (0)
-#define GS_STORE(RA_, RB_, BS_, buf)                                                           \
+#define GS_PUT(P_, v)                                                                          \
   do {                                                                                         \
+    bf16x4 h_, m_, l_;                                                                         \
+    split4((v), h_, m_, l_);                                                                   \
+    *reinterpret_cast<bf16x4*>(P_) = h_;                                                       \
+    *reinterpret_cast<bf16x4*>((P_) + PL) = m_;                                                \
+    *reinterpret_cast<bf16x4*>((P_) + 2 * PL) = l_;                                            \
+  } while (0)
+#define GS_STORE(RA_, RB_, buf, slab)                                                          \
+  do {                                                                                         \
+    const bool k_ = INNER || klo + (int64_t)(slab) * SK + sa_kq < K;                           \
     _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_) {                                        \
-      bf16x4 h_, m_, l_;                                                                       \
-      split4(RA_[i_], h_, m_, l_);                                                             \
-      __bf16* p_ = Ap + (buf) * 3 * PL + (sa_row + 64 * i_) * SP + sa_kq;                      \
-      *reinterpret_cast<bf16x4*>(p_) = h_;                                                     \
-      *reinterpret_cast<bf16x4*>(p_ + PL) = m_;                                                \
-      *reinterpret_cast<bf16x4*>(p_ + 2 * PL) = l_;                                            \
-    }                                                                                          \
-    if (B_KCONTIG) {                                                                           \
-      _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_) {                                      \
-        bf16x4 h_, m_, l_;                                                                     \
-        split4(RB_[i_], h_, m_, l_);                                                           \
-        __bf16* p_ = Bp + (buf) * 3 * PL + (sa_row + 64 * i_) * SP + sa_kq;                    \
-        *reinterpret_cast<bf16x4*>(p_) = h_;                                                   \
-        *reinterpret_cast<bf16x4*>(p_ + PL) = m_;                                              \
-        *reinterpret_cast<bf16x4*>(p_ + 2 * PL) = l_;                                          \
-      }                                                                                        \
-    } else {                                                                                   \
-      _Pragma("unroll") for (int q_ = 0; q_ < KPT / 4; ++q_) {                                 \
-        bf16x4 h_, m_, l_;                                                                     \
-        split4(make_float4(BS_[4 * q_], BS_[4 * q_ + 1], BS_[4 * q_ + 2], BS_[4 * q_ + 3]),    \
-               h_, m_, l_);                                                                    \
-        __bf16* p_ = Bp + (buf) * 3 * PL + sb_n * SP + sb_k + 4 * q_;                          \
-        *reinterpret_cast<bf16x4*>(p_) = h_;                                                   \
-        *reinterpret_cast<bf16x4*>(p_ + PL) = m_;                                              \
-        *reinterpret_cast<bf16x4*>(p_ + 2 * PL) = l_;                                          \
-      }                                                                                        \
+      const int o_ = (buf) * 3 * PL + (sa_row + 64 * i_) * SP + sa_kq;                         \
+      GS_PUT(Ap + o_, keep4(RA_[i_], k_));                                                     \
+      GS_PUT(Bp + o_, keep4(RB_[i_], k_));                                                     \
     }                                                                                          \
   } while (0)
     // The six cross products whose pieces sum to at most 2⁻¹⁶ relative (the
@@ -416,51 +445,55 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
       if (r_ % 4 == 3) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0); /* VMEM read */      \
     }                                                                                          \
   } while (0)
-#define GS_STEP(t, RA_, RB_, BS_)                                                              \
+#define GS_STEP(t, RA_, RB_)                                                                   \
   do {                                                                                         \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     if ((t) < nk) GS_MMA((t) & 1);                                                             \
-    GS_STORE(RA_, RB_, BS_, ((t) + 1) & 1);                                                    \
-    GS_LOAD(RA_, RB_, BS_, (t) + 5);                                                           \
+    GS_STORE(RA_, RB_, ((t) + 1) & 1, (t) + 1);                                                \
+    GS_LOAD(RA_, RB_, (t) + 5);                                                                \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     __syncthreads();                                                                           \
   } while (0)
     // A step known to be inside the K range: one basic block, interleaved.
-#define GS_STEP_IN(t, RA_, RB_, BS_)                                                           \
+#define GS_STEP_IN(t, RA_, RB_)                                                                \
   do {                                                                                         \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     GS_MMA((t) & 1);                                                                           \
-    GS_STORE(RA_, RB_, BS_, ((t) + 1) & 1);                                                    \
-    GS_LOAD(RA_, RB_, BS_, (t) + 5);                                                           \
+    GS_STORE(RA_, RB_, ((t) + 1) & 1, (t) + 1);                                                \
+    GS_LOAD(RA_, RB_, (t) + 5);                                                                \
     GS_PATTERN();                                                                              \
     __builtin_amdgcn_sched_barrier(0);                                                         \
     __syncthreads();                                                                           \
   } while (0)
-    const int nk = K > klo ? (int)cdiv(K - klo, (int64_t)SK) : 0;
+    auto loop = [&](auto inner_tag) __attribute__((always_inline)) {
+      constexpr bool INNER = decltype(inner_tag)::value;
+      GS_LOAD(ra0, rb0, 0);
+      GS_LOAD(ra1, rb1, 1);
+      GS_LOAD(ra2, rb2, 2);
+      GS_LOAD(ra3, rb3, 3);
+      GS_STORE(ra0, rb0, 0, 0);
+      GS_LOAD(ra0, rb0, 4);
+      __syncthreads();
+      int kt = 0;
+      for (; kt + 4 <= nk; kt += 4) {
+        GS_STEP_IN(kt, ra1, rb1);
+        GS_STEP_IN(kt + 1, ra2, rb2);
+        GS_STEP_IN(kt + 2, ra3, rb3);
+        GS_STEP_IN(kt + 3, ra0, rb0);
+      }
+      if (kt < nk) {
+        GS_STEP(kt, ra1, rb1);
+        GS_STEP(kt + 1, ra2, rb2);
+        GS_STEP(kt + 2, ra3, rb3);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
     if (nk > 0) {
-      GS_LOAD(ra0, rb0, bs0, 0);
-      GS_STORE(ra0, rb0, bs0, 0);
-      GS_LOAD(ra1, rb1, bs1, 1);
-      GS_LOAD(ra2, rb2, bs2, 2);
-      GS_LOAD(ra3, rb3, bs3, 3);
-      GS_LOAD(ra0, rb0, bs0, 4);
+      if (VEC && ((K - klo) & (SK - 1)) == 0) loop(BoolTag<VEC>{});
+      else loop(BoolTag<false>{});
     }
-    __syncthreads();
-    int kt = 0;
-    for (; kt + 4 <= nk; kt += 4) {
-      GS_STEP_IN(kt, ra1, rb1, bs1);
-      GS_STEP_IN(kt + 1, ra2, rb2, bs2);
-      GS_STEP_IN(kt + 2, ra3, rb3, bs3);
-      GS_STEP_IN(kt + 3, ra0, rb0, bs0);
-    }
-    if (kt < nk) {
-      GS_STEP(kt, ra1, rb1, bs1);
-      GS_STEP(kt + 1, ra2, rb2, bs2);
-      GS_STEP(kt + 2, ra3, rb3, bs3);
-      GS_STEP(kt + 3, ra0, rb0, bs0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
 #undef GS_LOAD
+#undef GS_PUT
 #undef GS_STORE
 #undef GS_MMA
 #undef GS_STEP
@@ -473,7 +506,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
     const int nk2 = (nk + 1) & ~1;
     if (nk2 > 0) {
       GF_LOAD(xa, xb, 0);
-      GF_STORE(xa, xb, 0);
+      GF_STORE(xa, xb, 0, 0);
       GF_LOAD(xa, xb, 1);
       GF_LOAD(ya, yb, 2);
     }
@@ -481,13 +514,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
     for (int kt = 0; kt < nk2; kt += 2) {
       __builtin_amdgcn_sched_barrier(0);
       if (SPLIT) GF_MMA_SPLIT(0); else GF_MMA(0);  // slab kt
-      GF_STORE(xa, xb, 1);    // slab kt+1
+      GF_STORE(xa, xb, 1, kt + 1);
       GF_LOAD(xa, xb, kt + 3);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
       if (SPLIT) GF_MMA_SPLIT(1); else GF_MMA(1);  // slab kt+1
-      GF_STORE(ya, yb, 0);    // slab kt+2
+      GF_STORE(ya, yb, 0, kt + 2);
       GF_LOAD(ya, yb, kt + 4);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
@@ -592,11 +625,7 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
 
   auto ld4 = [&](const float* base, int64_t ld, int64_t r, int64_t c, int64_t R, int64_t Ccols) {
     if (VEC) {
-      const bool ok = r < R && c < Ccols;
-      const uint4 w = *reinterpret_cast<const uint4*>(base + (ok ? r * ld + c : 0));
-      const uint32_t m = ok ? 0xffffffffu : 0u;
-      return make_float4(__uint_as_float(w.x & m), __uint_as_float(w.y & m),
-                         __uint_as_float(w.z & m), __uint_as_float(w.w & m));
+      return *reinterpret_cast<const float4*>(base + (r < R ? r : R - 1) * ld + (c < Ccols ? c : 0));
     }
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (r < R) {
@@ -610,16 +639,32 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
   };
 
   // Stage = 16 k: row r of a tile as four 4-k quads; thread tid holds quads
-  // (tid >> 2) + 128 i of both operands.
+  // (tid >> 2) + 128 i of both operands (loads, masks and INNER as in
+  // gemm_f32_kernel's split path).
   const int sa_row = tid >> 2, sa_kq = (tid & 3) * 4;
+  const int nk = (int)cdiv(K, (int64_t)SK);
+  const uint32_t oa0 = row_offset(m0, sa_row, M, g.lda, sa_kq);
+  const uint32_t oa1 = row_offset(m0, sa_row + 128, M, g.lda, sa_kq);
+  const uint32_t ob0 = row_offset(n0, sa_row, N, g.ldb, sa_kq);
+  const uint32_t ob1 = row_offset(n0, sa_row + 128, N, g.ldb, sa_kq);
+  const char* const ua = reinterpret_cast<const char*>(A + m0 * g.lda);
+  const char* const ub = reinterpret_cast<const char*>(B + n0 * g.ldb);
   float4 xa0, xa1, xb0, xb1, ya0, ya1, yb0, yb1;
 #define S2_LOAD(R, st)                                                                         \
   do {                                                                                         \
-    const int64_t k0_ = (int64_t)(st) * SK;                                                    \
-    R##a0 = ld4(A, g.lda, m0 + sa_row, k0_ + sa_kq, M, K);                                     \
-    R##a1 = ld4(A, g.lda, m0 + sa_row + 128, k0_ + sa_kq, M, K);                               \
-    R##b0 = ld4(B, g.ldb, n0 + sa_row, k0_ + sa_kq, N, K);                                     \
-    R##b1 = ld4(B, g.ldb, n0 + sa_row + 128, k0_ + sa_kq, N, K);                               \
+    if constexpr (INNER) {                                                                     \
+      const int64_t sl_ = (int64_t)((st) < nk ? (st) : nk - 1) * (SK * 4);                     \
+      R##a0 = *reinterpret_cast<const float4*>(ua + sl_ + oa0);                                \
+      R##a1 = *reinterpret_cast<const float4*>(ua + sl_ + oa1);                                \
+      R##b0 = *reinterpret_cast<const float4*>(ub + sl_ + ob0);                                \
+      R##b1 = *reinterpret_cast<const float4*>(ub + sl_ + ob1);                                \
+    } else {                                                                                   \
+      const int64_t k0_ = (int64_t)(st) * SK;                                                  \
+      R##a0 = ld4(A, g.lda, m0 + sa_row, k0_ + sa_kq, M, K);                                   \
+      R##a1 = ld4(A, g.lda, m0 + sa_row + 128, k0_ + sa_kq, M, K);                             \
+      R##b0 = ld4(B, g.ldb, n0 + sa_row, k0_ + sa_kq, N, K);                                   \
+      R##b1 = ld4(B, g.ldb, n0 + sa_row + 128, k0_ + sa_kq, N, K);                             \
+    }                                                                                          \
   } while (0)
 #define S2_PUT(P, buf, row, v)                                                                 \
   do {                                                                                         \
@@ -630,12 +675,13 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
     *reinterpret_cast<bf16x4*>(&P[(buf)][1][o_]) = m_;                                         \
     *reinterpret_cast<bf16x4*>(&P[(buf)][2][o_]) = l_;                                         \
   } while (0)
-#define S2_STORE(R, buf)                                                                       \
+#define S2_STORE(R, buf, st)                                                                   \
   do {                                                                                         \
-    S2_PUT(Ap, buf, sa_row, R##a0);                                                            \
-    S2_PUT(Ap, buf, sa_row + 128, R##a1);                                                      \
-    S2_PUT(Bp, buf, sa_row, R##b0);                                                            \
-    S2_PUT(Bp, buf, sa_row + 128, R##b1);                                                      \
+    const bool k_ = INNER || (int64_t)(st) * SK + sa_kq < K;                                   \
+    S2_PUT(Ap, buf, sa_row, keep4(R##a0, k_));                                                 \
+    S2_PUT(Ap, buf, sa_row + 128, keep4(R##a1, k_));                                           \
+    S2_PUT(Bp, buf, sa_row, keep4(R##b0, k_));                                                 \
+    S2_PUT(Bp, buf, sa_row + 128, keep4(R##b1, k_));                                           \
   } while (0)
 
   f32x16 acc[4][2];
@@ -676,29 +722,33 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
   // Stage t is multiplied out of buffer t&1 while stage t+1 goes from its
   // register set to the other buffer and that set loads stage t+3; stages
   // past K load zeros and skip their MFMAs.  One barrier per stage.
-  const int nk = (int)cdiv(K, (int64_t)SK);
-  S2_LOAD(x, 0);
-  S2_STORE(x, 0);
-  S2_LOAD(x, 1);
-  S2_LOAD(y, 2);
-  __syncthreads();
-  for (int kt = 0; kt < nk; kt += 2) {
-    __builtin_amdgcn_sched_barrier(0);
-    S2_MMA(0);
-    S2_STORE(x, 1);
-    S2_LOAD(x, kt + 3);
-    __builtin_amdgcn_sched_barrier(0);
+  auto loop = [&](auto inner_tag) __attribute__((always_inline)) {
+    constexpr bool INNER = decltype(inner_tag)::value;
+    S2_LOAD(x, 0);
+    S2_STORE(x, 0, 0);
+    S2_LOAD(x, 1);
+    S2_LOAD(y, 2);
     __syncthreads();
-    if (kt + 1 < nk) {
+    for (int kt = 0; kt < nk; kt += 2) {
       __builtin_amdgcn_sched_barrier(0);
-      S2_MMA(1);
-      S2_STORE(y, 0);
-      S2_LOAD(y, kt + 4);
+      S2_MMA(0);
+      S2_STORE(x, 1, kt + 1);
+      S2_LOAD(x, kt + 3);
       __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
+      if (kt + 1 < nk) {
+        __builtin_amdgcn_sched_barrier(0);
+        S2_MMA(1);
+        S2_STORE(y, 0, kt + 2);
+        S2_LOAD(y, kt + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+      }
     }
-  }
-  __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (VEC && (K & (SK - 1)) == 0) loop(BoolTag<VEC>{});
+  else loop(BoolTag<false>{});
 #undef S2_LOAD
 #undef S2_PUT
 #undef S2_STORE
@@ -785,6 +835,11 @@ void launch_gemm(hipStream_t stream, const GemmF32& g, bool vec, int64_t nz, boo
   }
 }
 
+// Share of the workgroup slots (`slots` at a time) that n workgroups keep busy.
+double round_fill(int64_t n, int64_t slots) {
+  return (double)n / (double)(cdiv(n, slots) * slots);
+}
+
 }  // namespace
 
 int gemm_f32(hipStream_t stream, const GemmF32& g) {
@@ -806,7 +861,7 @@ int gemm_f32(hipStream_t stream, const GemmF32& g) {
   };
   // ... and whole 16-byte chunks along k (and along n for B given K×N).
   const bool vec = al(g.A, g.lda, g.sA, g.sA2) && al(g.B, g.ldb, g.sB, g.sB2) && g.K % 4 == 0 &&
-                   (g.b_kcontig || g.N % 4 == 0);
+                   (g.b_kcontig || g.N % 4 == 0) && g.lda < (1 << 22) && g.ldb < (1 << 22);
   // 128×128 tiles unless that grid would leave most of the 256 CUs (two
   // workgroups each) idle.
   // Products with K >= 128 run on the bf16 matrix cores from split operands
@@ -817,12 +872,23 @@ int gemm_f32(hipStream_t stream, const GemmF32& g) {
               "gemm_f32: ldb %lld too large for the split path's 32-bit row offsets",
               (long long)g.ldb);
   const int64_t t256 = cdiv(g.M, (int64_t)S2T) * cdiv(g.N, (int64_t)S2T);
-  if (split && g.b_kcontig && g.tri == 0 && g.K >= 384 && t256 * nz >= 256) {
+  // 256×256 tiles (one workgroup per CU) against 128×128 (two): the larger
+  // tile is 6 to 10 % faster per full round of workgroups, so it is taken
+  // unless its last round wastes more than that (MI355X, K = 512: 4096×4096
+  // 102 against 109 us at one full round of 256 tiles, 13824×13824 1100
+  // against 1169; 4096×13312, 3.25 rounds, 349 against 323).
+  const double fill256 = round_fill(t256 * nz, 256), fill128 = round_fill(t128 * nz, 512);
+  // Long products with few rows (the factor's inverse rows) take 128×128
+  // tiles from one workgroup per CU on: 512×8192×8192 404 against 470 us on
+  // 64×64 tiles, 512×13824×13824 1049 against 1340, 512×6144×6144 equal.
+  const bool long_k = split && g.b_kcontig && g.K >= 2048 && t128 * nz >= 224;
+  if (split && g.b_kcontig && g.tri == 0 && g.K >= 384 && t256 * nz >= 256 &&
+      1.07 * fill256 >= fill128) {
     const int64_t tm = cdiv(g.M, (int64_t)S2T), tn = cdiv(g.N, (int64_t)S2T);
     const dim3 grid((unsigned)(tm * tn), 1, (unsigned)nz);
     if (vec) hipLaunchKernelGGL(gemm_s256_kernel<true>, grid, dim3(512), 0, stream, g, tm, tn);
     else hipLaunchKernelGGL(gemm_s256_kernel<false>, grid, dim3(512), 0, stream, g, tm, tn);
-  } else if (t128 * nz >= 512) {
+  } else if (t128 * nz >= 512 || long_k) {
     launch_gemm<128>(stream, g, vec, nz, split);
   } else {
     launch_gemm<64>(stream, g, vec, nz, split);
