@@ -713,6 +713,8 @@ __device__ __forceinline__ float group_bcast(float v, int o) {
   }
 }
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 template <int V, int L, bool F, bool SBM = false>
 __global__ __launch_bounds__(256) void sweep4_kernel(SweepArgs a) {
   constexpr int PW = 32, RW = 256 / L;  // panel width, rows per workgroup
@@ -1129,47 +1131,62 @@ __global__ __launch_bounds__(256) void sweep4_kernel(SweepArgs a) {
   }
     if (SBM && bi + 1 < nblk) {
       // Near tail of the super-block: W[row, c] −= Σ_k e_k·U[cofs + k, c] for
-      // the columns c of the later blocks, 64 at a time (the triangle's LDS
-      // holds the U slab, k-major), four consecutive columns per lane.
-      float* Wr = a.Wsb + b * a.wb + r * a.wr;
-      const float* Ub = a.U + b * a.ub + cofs * a.uj;
-      // A thread's eight 16-byte pieces of a slab are all loaded before any
-      // is stored: one memory round trip per slab, not eight.
-      static_assert(kMaxBlock * 16 == 8 * 256, "a slab is eight 16-byte pieces per thread");
-      // thread tid's piece i: row k = tid/16 + 16i of the slab, columns 4·(tid%16)..+3
-      const int k0 = tid >> 4, c4 = (tid & 15) * 4;
-      for (int c0 = (int)cofs + kMaxBlock; c0 < nblk * kMaxBlock; c0 += 64) {
-        const float* us = Ub + (int64_t)k0 * a.uj + c0 + c4;
-        const int64_t st16 = 16 * a.uj;
-#define G2_LDU(i) const float4 u##i = *reinterpret_cast<const float4*>(us + (i) * st16)
-        G2_LDU(0); G2_LDU(1); G2_LDU(2); G2_LDU(3); G2_LDU(4); G2_LDU(5); G2_LDU(6); G2_LDU(7);
-#undef G2_LDU
-        __syncthreads();  // the sweep's (or the previous slab's) LDS reads are done
-        float* ud = &Us[k0 * 64 + c4];
-#define G2_STU(i) *reinterpret_cast<float4*>(ud + (i) * 16 * 64) = u##i
-        G2_STU(0); G2_STU(1); G2_STU(2); G2_STU(3); G2_STU(4); G2_STU(5); G2_STU(6); G2_STU(7);
-#undef G2_STU
-        __syncthreads();
-        if (act) {
-          float4 w = *reinterpret_cast<const float4*>(Wr + c0 + 4 * sub);
-          float t[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 4
-          for (int k = 0; k < kMaxBlock; k += 2) {
+      // the columns c of the later blocks, on v_mfma_f32_16x16x4_f32, whose
+      // four k are the ascending chain of four fused multiply-adds bit for bit
+      // (measured on MI355X): one chain over the even k and one over the odd,
+      // added at the end.  A wave takes all 16 rows of 32 columns at a time,
+      // as two tiles (even and odd columns, so that a lane's loads, of U as of
+      // W, are two consecutive floats).  No two waves read the same part of U,
+      // so it goes from memory to the fragments without LDS, half a chunk (64
+      // k) ahead.  MI355X, R = 4096, C = 4096, in the loop: 127 us per launch
+      // with the U slabs staged in LDS and fp32 FMAs, 107 so.
+      __syncthreads();  // every row's errors are in e_s
+      constexpr int HK = 16;  // loads per half: k = 64·half + 8·(i / 2) + 2·g + i % 2
+      const int lane = tid & 63, g = lane >> 4, nn = lane & 15;
+      float* Wr = a.Wsb + b * a.wb + ((int64_t)blockIdx.x * RW + 4 * g) * a.wr + 2 * nn;
+      const float* Ub = a.U + b * a.ub + (cofs + 2 * g) * a.uj + 2 * nn;
+      const int64_t left = a.R - ((int64_t)blockIdx.x * RW + 4 * g);  // rows of this lane in range
+      float ae[2 * HK];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const float e = e_s[(k + h) * RW + rr];
-              const float4 u = *reinterpret_cast<const float4*>(&Us[(k + h) * 64 + 4 * sub]);
-              t[h][0] = __builtin_fmaf(e, u.x, t[h][0]);
-              t[h][1] = __builtin_fmaf(e, u.y, t[h][1]);
-              t[h][2] = __builtin_fmaf(e, u.z, t[h][2]);
-              t[h][3] = __builtin_fmaf(e, u.w, t[h][3]);
-            }
-          }
-          w.x = __fsub_rn(w.x, __fadd_rn(t[0][0], t[1][0]));
-          w.y = __fsub_rn(w.y, __fadd_rn(t[0][1], t[1][1]));
-          w.z = __fsub_rn(w.z, __fadd_rn(t[0][2], t[1][2]));
-          w.w = __fsub_rn(w.w, __fadd_rn(t[0][3], t[1][3]));
-          *reinterpret_cast<float4*>(Wr + c0 + 4 * sub) = w;
+      for (int i = 0; i < 2 * HK; ++i) ae[i] = e_s[(8 * (i >> 1) + 2 * g + (i & 1)) * RW + nn];
+      float2 ul[HK], uh[HK];
+      auto load_half = [&](float2 (&u)[HK], int half, int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < HK; ++i)
+          u[i] = *reinterpret_cast<const float2*>(
+              Ub + (int64_t)(64 * half + 8 * (i >> 1) + (i & 1)) * a.uj + c0);
+      };
+      const int cend = nblk * kMaxBlock;
+      int c0 = (int)cofs + kMaxBlock + 32 * (tid >> 6);
+      load_half(ul, 0, c0);
+      load_half(uh, 1, c0);
+#pragma clang loop unroll(disable)
+      for (; c0 < cend; c0 += 4 * 32) {
+        const int cn = c0 + 4 * 32 < cend ? c0 + 4 * 32 : c0;  // the next chunk (or this one again)
+        float2 w[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          w[v] = *reinterpret_cast<const float2*>(Wr + (v < left ? v : 0) * a.wr + c0 +
+                                                  (left > 0 ? 0 : -4 * g * a.wr));
+        f32x4 t[2][2] = {{{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}},
+                         {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}};
+#pragma unroll
+        for (int i = 0; i < HK; ++i) {
+          t[i & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ae[i], ul[i].x, t[i & 1][0], 0, 0, 0);
+          t[i & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ae[i], ul[i].y, t[i & 1][1], 0, 0, 0);
+        }
+        load_half(ul, 0, cn);
+#pragma unroll
+        for (int i = 0; i < HK; ++i) {
+          t[i & 1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ae[HK + i], uh[i].x, t[i & 1][0], 0, 0, 0);
+          t[i & 1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ae[HK + i], uh[i].y, t[i & 1][1], 0, 0, 0);
+        }
+        load_half(uh, 1, cn);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          w[v].x = __fsub_rn(w[v].x, __fadd_rn(t[0][0][v], t[1][0][v]));
+          w[v].y = __fsub_rn(w[v].y, __fadd_rn(t[0][1][v], t[1][1][v]));
+          if (v < left) *reinterpret_cast<float2*>(Wr + v * a.wr + c0) = w[v];
         }
       }
     }
