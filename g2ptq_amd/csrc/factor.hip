@@ -370,11 +370,13 @@ __global__ __launch_bounds__(256) void panel_step_kernel(PanelArgs p) {
   }
 }
 
-// The panel's last column block [j, pe): workgroup t owns rows
-// [k + 64(t + 1), +64).  Rows below the panel get their TRSM for this block in
-// place (L = Â·X_jjᵀ; nothing else reads these raw values); every row gets the
-// panel buffer's L columns left of its own diagonal block (or of this block)
-// copied into Â.
+// The panel's last column block [j, pe): workgroups (t, ·, z) own rows
+// [k + 64(t + 1), +64).  z = 0: rows below the panel get their TRSM for this
+// block in place (L = Â·X_jjᵀ; nothing else reads these raw values).  z > 0:
+// the panel buffer's columns [64(z − 1), +64), where they are left of the rows'
+// own diagonal block (or of this block), are copied into Â.  Latency-bound on
+// the panel chain: one workgroup per row block doing both took 20 µs at
+// 3584 rows, 9 µs split by columns.
 __global__ __launch_bounds__(256) void panel_finish_kernel(PanelArgs p) {
   __shared__ __attribute__((aligned(16))) float Xj[64 * SLP];
   __shared__ __attribute__((aligned(16))) float Ai[64 * SLP];
@@ -383,44 +385,28 @@ __global__ __launch_bounds__(256) void panel_finish_kernel(PanelArgs p) {
   const int64_t C = p.C;
   const int64_t R0 = p.k + 64 * ((int64_t)blockIdx.x + 1);
   float* Wb = p.WA + b * C * C;
-  const float* Lb = p.Lp + b * C * NBO;
   const bool vec = (C & 3) == 0;
-  const int64_t cend = (R0 < p.pe ? R0 : p.j) - p.k;  // buffer columns to copy
-  {
-    const int nq = (int)(cend >> 2);  // cend is a multiple of 64
-    // eight 16-byte pieces per thread and pass, all loaded before any is stored
-    constexpr int U = 8;
-    for (int q0 = threadIdx.x; q0 < 64 * nq; q0 += 256 * U) {
-      float4 x[U];
+  if (blockIdx.z > 0) {
+    const int64_t c0 = 64 * ((int64_t)blockIdx.z - 1);
+    if (c0 >= (R0 < p.pe ? R0 : p.j) - p.k) return;  // both ends multiples of 64
+    const float* src = p.Lp + b * C * NBO + c0 + (threadIdx.x & 15) * 4;
+    float* dst = Wb + p.k + c0 + (threadIdx.x & 15) * 4;
+    const int64_t r0 = R0 + (threadIdx.x >> 4);
+    float4 x[4];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + 256 * u;
-        const int64_t r = R0 + q / nq;
-        const int64_t c4 = (int64_t)(q % nq) * 4;
-        if (q < 64 * nq && r < C) {
-          const float* s = Lb + r * NBO + c4;
-          if (vec) {
-            x[u] = *reinterpret_cast<const float4*>(s);
-          } else {
-            x[u] = make_float4(s[0], s[1], s[2], s[3]);
-          }
-        }
-      }
+    for (int q = 0; q < 4; ++q)
+      x[q] = *reinterpret_cast<const float4*>(src + std::min(r0 + 16 * q, C - 1) * NBO);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 + 256 * u;
-        const int64_t r = R0 + q / nq;
-        const int64_t c4 = (int64_t)(q % nq) * 4;
-        if (q < 64 * nq && r < C) {
-          float* d = Wb + r * C + p.k + c4;
-          if (vec) {
-            *reinterpret_cast<float4*>(d) = x[u];
-          } else {
-            d[0] = x[u].x; d[1] = x[u].y; d[2] = x[u].z; d[3] = x[u].w;
-          }
-        }
+    for (int q = 0; q < 4; ++q) {
+      if (r0 + 16 * q >= C) break;
+      float* d = dst + (r0 + 16 * q) * C;
+      if (vec) {
+        *reinterpret_cast<float4*>(d) = x[q];
+      } else {
+        d[0] = x[q].x; d[1] = x[q].y; d[2] = x[q].z; d[3] = x[q].w;
       }
     }
+    return;
   }
   if (R0 < p.pe) return;
   {
@@ -674,13 +660,16 @@ extern "C" int g2ptq_inv_chol_upper(void* stream, const float* H, int64_t B, int
         // TRSM of the rows below the panel for its last block; the panel
         // buffer's L into Â
         pa.pot_nb = 0;
-        hipLaunchKernelGGL(panel_finish_kernel, dim3((unsigned)cdiv(C - k - NB, 64), (unsigned)B),
+        hipLaunchKernelGGL(panel_finish_kernel,
+                           dim3((unsigned)cdiv(C - k - NB, 64), (unsigned)B,
+                                (unsigned)(1 + (j - k) / 64)),
                            dim3(256), 0, s, pa);
         G2PTQ_LAUNCHED();
       }
     }
-    G2PTQ_HIP(hipEventRecord(side.factored, s));
-    G2PTQ_HIP(hipStreamWaitEvent(side.stream2, side.factored, 0));
+    return G2PTQ_OK;
+  };
+  auto invert_panel = [&](int64_t k, int64_t kb) -> int {
     inv_pending = true;
     G2PTQ_TRY(trtri_levels(side.stream2, k, kb, NB, NBO));
     if (k > 0) {
@@ -734,28 +723,33 @@ extern "C" int g2ptq_inv_chol_upper(void* stream, const float* H, int64_t B, int
       G2PTQ_TRY(syrk1(q, k, kb, c, std::min(c1, c + SYRK_CHUNK)));
     return G2PTQ_OK;
   };
-  G2PTQ_TRY(factor_panel(0, std::min<int64_t>(NBO, C)));
+  // Host order: what the chain waits for first (the next panel's own update,
+  // its factorization), the panel's inverse after it, so that a host that is
+  // not far ahead of the device delays only the work with slack (with the split panel
+  // finish, 4096x4096 GPTQ layer 3.31 -> 3.13 ms).
   int pend = -1;  // ping-pong slot of the latest trailing update on the side stream
+  G2PTQ_TRY(factor_panel(0, std::min<int64_t>(NBO, C)));
   for (int64_t k = 0, p = 0; k < C; k += NBO, ++p) {
     const int64_t kb = std::min<int64_t>(NBO, C - k);
     const int64_t next = k + kb;
-    if (next >= C) break;
-    const int64_t nb2 = std::min<int64_t>(NBO, C - next);
-    if (next + nb2 < C) {  // trailing part beyond the next panel, on the side stream
-      G2PTQ_HIP(hipEventRecord(side.factored, s));
-      G2PTQ_HIP(hipStreamWaitEvent(side.stream, side.factored, 0));
-      G2PTQ_TRY(syrk(side.stream, k, kb, next + nb2, C));
-    }
-    // The next panel's columns also received the previous trailing update.
-    if (pend >= 0) G2PTQ_HIP(hipStreamWaitEvent(s, side.done[pend], 0));
-    if (next + nb2 < C) {
-      pend = (int)(p & 1);
-      G2PTQ_HIP(hipEventRecord(side.done[pend], side.stream));
-    } else {
+    const int64_t nb2 = std::min<int64_t>(NBO, C - next);  // <= 0 after the last panel
+    G2PTQ_HIP(hipEventRecord(side.factored, s));  // panel k
+    G2PTQ_HIP(hipStreamWaitEvent(side.stream2, side.factored, 0));
+    if (next < C) {
+      const bool far = next + nb2 < C;  // trailing part beyond the next panel: side stream
+      if (far) G2PTQ_HIP(hipStreamWaitEvent(side.stream, side.factored, 0));
+      // The next panel's columns also received the previous trailing update.
+      if (pend >= 0) G2PTQ_HIP(hipStreamWaitEvent(s, side.done[pend], 0));
+      G2PTQ_TRY(syrk(s, k, kb, next, next + nb2));
       pend = -1;
+      if (far) {
+        G2PTQ_TRY(syrk(side.stream, k, kb, next + nb2, C));
+        pend = (int)(p & 1);
+        G2PTQ_HIP(hipEventRecord(side.done[pend], side.stream));
+      }
+      G2PTQ_TRY(factor_panel(next, nb2));
     }
-    G2PTQ_TRY(syrk(s, k, kb, next, next + nb2));
-    G2PTQ_TRY(factor_panel(next, nb2));
+    G2PTQ_TRY(invert_panel(k, kb));
   }
   if (pend >= 0) G2PTQ_HIP(hipStreamWaitEvent(s, side.done[pend], 0));
 
