@@ -35,12 +35,36 @@ __global__ void triu1_kernel(float* t, int64_t C) {
 // factor as N×K rows, k-contiguous, which the GEMM stages and splits once
 // per workgroup (faster than splitting a K×N operand per wave).
 __global__ __launch_bounds__(256) void transpose_upper_kernel(const float* __restrict__ U,
-                                                              int64_t C, float* __restrict__ Ut) {
+                                                              int64_t C, float* __restrict__ Ut,
+                                                              bool vec) {
   const int64_t bi = blockIdx.y, bj = blockIdx.x, b = blockIdx.z;
   if (bi > bj) return;
   __shared__ float t[64][65];
   const float* Ub = U + b * C * C;
   float* Tb = Ut + b * C * C;
+  if (vec) {
+    const int c4 = (threadIdx.x & 15) * 4, r0 = threadIdx.x >> 4;
+    float4 x[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)  // addresses held inside the matrix
+      x[q] = *reinterpret_cast<const float4*>(Ub + std::min(bi * 64 + r0 + 16 * q, C - 1) * C +
+                                              std::min(bj * 64 + c4, C - 4));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float* d = &t[r0 + 16 * q][c4];
+      d[0] = x[q].x; d[1] = x[q].y; d[2] = x[q].z; d[3] = x[q].w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = r0 + 16 * q;
+      const int64_t j = bj * 64 + r, i = bi * 64 + c4;
+      if (i < C && j < C)
+        *reinterpret_cast<float4*>(Tb + j * C + i) =
+            make_float4(t[c4][r], t[c4 + 1][r], t[c4 + 2][r], t[c4 + 3][r]);
+    }
+    return;
+  }
   const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
@@ -256,7 +280,7 @@ static int compensate_impl(hipStream_t s, int variant, int64_t B, int64_t R, int
   if (Ut) {
     const unsigned nt = (unsigned)cdiv(C, (int64_t)64);
     hipLaunchKernelGGL(transpose_upper_kernel, dim3(nt, nt, (unsigned)B), dim3(256), 0, s, U, C,
-                       Ut);
+                       Ut, C % 4 == 0 && ((uintptr_t)U & 15) == 0 && ((uintptr_t)Ut & 15) == 0);
     G2PTQ_LAUNCHED();
   }
 
