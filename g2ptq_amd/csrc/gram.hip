@@ -872,6 +872,25 @@ __global__ __launch_bounds__(NTH) void wgram_kernel(G2Args a) {
       I, J, diag, wm, wn, lh, lr);
 }
 
+// sum[k] += a thread's row k (16 rows apart) of N consecutive splits, in split
+// order, all of them loaded first.
+template <int N>
+__device__ __forceinline__ void reduce_splits(float4 (&sum)[4], const float* p0) {
+  float4 p[N][4];
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      p[u][k] = *reinterpret_cast<const float4*>(p0 + u * (int64_t)(TT * TT) + 16 * k * TT);
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      sum[k].x += p[u][k].x; sum[k].y += p[u][k].y;
+      sum[k].z += p[u][k].z; sum[k].w += p[u][k].w;
+    }
+}
+
 // H[I,J] = beta·H + alpha·Σ_s partial_s (fixed order), mirrored for symmetric
 // products.  One workgroup reduces a 64×64 block of a tile: rows are read and
 // written as 16-byte vectors, and the mirror goes through an LDS transpose so
@@ -897,37 +916,36 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
   const int cq = tid & 15, r0 = tid >> 4;
   const int64_t ti = I * TT + bi * 64, tj = J * TT + bj * 64;  // global block origin
   const bool vec = (a.ldh & 3) == 0;
-  // The thread's four rows of the block, four splits at a time: sixteen
-  // 16-byte loads in flight (one at a time left the launch waiting for
-  // memory: C = 4096, 15 splits, MI355X, 147 us so and 125 now, 4.8 TB/s),
-  // each row summed in split order.
+  const float* p0 = P + (bi * 64 + r0) * TT + bj * 64 + cq * 4;
+  // Symmetric products: the thread's four rows of the block, four splits at a
+  // time: sixteen 16-byte loads in flight (one at a time left the launch
+  // waiting for memory: C = 4096, 15 splits, MI355X, 147 us so and 125 now,
+  // 4.8 TB/s), each row summed in split order.  Full products have twice the
+  // blocks, enough to keep memory busy, and go row by row, so that one row's
+  // stores run beside the next one's loads (C = 1942: 15.7 us, 18.0 with all
+  // four rows first; C = 4096 the same either way).
   float4 sum[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) sum[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-  {
-    const float* p0 = P + (bi * 64 + r0) * TT + bj * 64 + cq * 4;
-    for (int sp = 0; sp < a.S; sp += 4) {
-      float4 p[4][4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float* pu = p0 + (sp + u < a.S ? sp + u : sp) * (int64_t)(TT * TT);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) p[u][k] = *reinterpret_cast<const float4*>(pu + 16 * k * TT);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (sp + u >= a.S) break;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          sum[k].x += p[u][k].x; sum[k].y += p[u][k].y;
-          sum[k].z += p[u][k].z; sum[k].w += p[u][k].w;
-        }
-      }
+  if (!FULL) {
+    int sp = 0;
+    for (; sp + 4 <= a.S; sp += 4) reduce_splits<4>(sum, p0 + sp * (int64_t)(TT * TT));
+    if (a.S & 2) {
+      reduce_splits<2>(sum, p0 + sp * (int64_t)(TT * TT));
+      sp += 2;
     }
+    if (a.S & 1) reduce_splits<1>(sum, p0 + sp * (int64_t)(TT * TT));
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int r = r0 + 16 * k;  // row within the block
+    if (FULL) {
+      for (int sp = 0; sp < a.S; ++sp) {
+        const float4 p =
+            *reinterpret_cast<const float4*>(p0 + sp * (int64_t)(TT * TT) + 16 * k * TT);
+        sum[k].x += p.x; sum[k].y += p.y; sum[k].z += p.z; sum[k].w += p.w;
+      }
+    }
     const int64_t i = ti + r, j = tj + cq * 4;
     float out[4] = {sum[k].x, sum[k].y, sum[k].z, sum[k].w};
     if (i < a.C) {
