@@ -108,6 +108,33 @@ struct SideStream {
 };
 int side_stream(hipStream_t caller, SideStream& out);
 
+// Launch of 256-thread workgroups over `rows` rows of `cells` items each: 2^shift
+// threads walk a row and the other 256 >> shift of a workgroup the rows below,
+// so that narrow rows fill their wavefronts too; at most about 16384 workgroups.
+struct RowLaunch {
+  dim3 grid;
+  int shift;
+};
+inline RowLaunch row_launch(int64_t cells, int64_t rows) {
+  int shift = 8;
+  while (shift > 0 && cells <= (int64_t)1 << (shift - 1)) --shift;
+  const int64_t gx = cdiv(cells, (int64_t)1 << shift);
+  int64_t gy = cdiv(rows, (int64_t)256 >> shift);
+  if (gy > 65535) gy = 65535;
+  if (gy > cdiv((int64_t)16384, gx)) gy = cdiv((int64_t)16384, gx);
+  return {dim3((unsigned)gx, (unsigned)(gy < 1 ? 1 : gy)), shift};
+}
+// A thread's item of its row, its first row and the distance to its next one.
+__device__ __forceinline__ int64_t row_cell(int shift) {
+  return ((int64_t)blockIdx.x << shift) + (threadIdx.x & ((1u << shift) - 1));
+}
+__device__ __forceinline__ int64_t row_first(int shift) {
+  return (int64_t)blockIdx.y * (256 >> shift) + (threadIdx.x >> shift);
+}
+__device__ __forceinline__ int64_t row_step(int shift) {
+  return (int64_t)gridDim.y * (256 >> shift);
+}
+
 // p[0..n) = v with a kernel (graph-capture safe, unlike hipMemsetAsync).
 int fill_f32(hipStream_t stream, float* p, int64_t n, float v);
 

@@ -423,19 +423,19 @@ __global__ __launch_bounds__(256) void fake_quantize_kernel(
 }
 
 // fake_quantize_kernel four columns at a time (groups of a multiple of four
-// columns, every row on a 16-byte boundary), a grid row per row: the same
-// operations per element, without a 64-bit division for each.  4096 × 4096 in
-// groups of 128, codes too, MI355X: 46-50 µs one column per thread,
-// 31 µs here (6.5 TB/s over x, the value and the code).
+// columns, every row on a 16-byte boundary), rows narrower than a workgroup
+// several to one: the same operations per element, without a 64-bit division
+// for each.  4096 × 4096 in groups of 128, codes too, MI355X: 46-50 µs one
+// column per thread, 31 µs here (6.5 TB/s over x, the value and the code).
 __global__ __launch_bounds__(256) void fake_quantize_vec_kernel(
     const float* __restrict__ x, int64_t rows, int64_t cols, int64_t ldx, int64_t gsize,
     const float* __restrict__ scale, const float* __restrict__ zero, int64_t ldp, int maxq,
-    float* q_out, int64_t ldq, float* int_out, int64_t ldi) {
+    float* q_out, int64_t ldq, float* int_out, int64_t ldi, int shift) {
   const float minq = (float)(-(maxq + 1)), fmaxq = (float)maxq;
-  const int64_t c = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const int64_t c = row_cell(shift) * 4;
   if (c >= cols) return;
   const int64_t gidx = gsize > 0 ? (uint32_t)c / (uint32_t)gsize : 0;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+  for (int64_t r = row_first(shift); r < rows; r += row_step(shift)) {
     const float s = scale[r * ldp + gidx], z = zero[r * ldp + gidx];
     const float4 x4 = *reinterpret_cast<const float4*>(x + r * ldx + c);
     const float v[4] = {x4.x, x4.y, x4.z, x4.w};
@@ -1404,12 +1404,10 @@ extern "C" int g2ptq_fake_quantize(void* stream, const float* x, int64_t rows, i
   if (cols % 4 == 0 && (groupsize <= 0 || groupsize % 4 == 0) && ldx % 4 == 0 && ldq % 4 == 0 &&
       aligned16(x) && aligned16(q_out) && (!int_out || (ldi % 4 == 0 && aligned16(int_out))) &&
       cols < (1ll << 31) && groupsize < (1ll << 31)) {
-    const int64_t gx = cdiv(cols / 4, (int64_t)256);
-    const int64_t gy = std::max<int64_t>(
-        1, std::min<int64_t>(std::min<int64_t>(rows, 65535), cdiv((int64_t)16384, gx)));
-    hipLaunchKernelGGL(fake_quantize_vec_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0,
-                       as_stream(stream), x, rows, cols, ldx, groupsize, scale, zero, ldp, maxq,
-                       q_out, ldq, int_out, ldi);
+    const RowLaunch rg = row_launch(cols / 4, rows);
+    hipLaunchKernelGGL(fake_quantize_vec_kernel, rg.grid, dim3(256), 0, as_stream(stream), x, rows,
+                       cols, ldx, groupsize, scale, zero, ldp, maxq, q_out, ldq, int_out, ldi,
+                       rg.shift);
     G2PTQ_LAUNCHED();
     return G2PTQ_OK;
   }
