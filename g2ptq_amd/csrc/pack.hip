@@ -56,19 +56,26 @@ __global__ void pack_codes_kernel(const float* __restrict__ codes, int64_t ldc, 
 }
 
 // pack_codes_kernel with the word's codes read as 16-byte pieces (32/bits a
-// multiple of four: bits 1, 2, 4, 7 and 8; rows on 16-byte boundaries), a
-// grid row per code row.  4096 × 4096 at 4 bits, MI355X: 37 µs with a word per thread
-// and 64-bit divisions, 14 µs here (4.7 TB/s).
-template <int PF>
+// multiple of four: bits 1, 2, 4, 7 and 8; rows on 16-byte boundaries), rows
+// narrower than a workgroup several to one (NARROW; a row index per workgroup
+// stays in scalar registers otherwise: 4096 × 4096 at 8 bits 13.5 µs so, 14.4
+// with one per thread).  4096 × 4096 at 4 bits, MI355X: 37 µs with a word per
+// thread and 64-bit divisions, 14 µs here (4.7 TB/s).
+template <int PF, bool NARROW>
 __global__ __launch_bounds__(256) void pack_codes_vec_kernel(const float* __restrict__ codes,
                                                              int64_t ldc, int64_t rows, int bits,
                                                              int32_t* __restrict__ packed,
-                                                             int64_t ldp, int64_t words) {
+                                                             int64_t ldp, int64_t words,
+                                                             int rowshift) {
+  // (a whole workgroup on a row: all from the block indices)
+  const int shift = NARROW ? rowshift : 8;
+  const int64_t first = NARROW ? row_first(shift) : blockIdx.y;
+  const int64_t step = NARROW ? row_step(shift) : gridDim.y;
   const int off = 1 << (bits - 1);
   const uint32_t mask = (1u << bits) - 1u;
-  const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t w = NARROW ? row_cell(shift) : (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (w >= words) return;
-  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+  for (int64_t r = first; r < rows; r += step) {
     const float4* src = reinterpret_cast<const float4*>(codes + r * ldc + w * PF);
     uint32_t acc = 0;
 #pragma unroll
@@ -84,17 +91,23 @@ __global__ __launch_bounds__(256) void pack_codes_vec_kernel(const float* __rest
 }
 
 // group_scale_kernel four columns at a time (groups of a multiple of four
-// columns, rows on 16-byte boundaries), a grid row per row.  4096 × 4096 in
-// groups of 128, MI355X: 35 µs one scale per thread, 14 µs here.
+// columns, rows on 16-byte boundaries), narrow rows as in pack_codes_vec_kernel.
+// 4096 × 4096 in groups of 128, MI355X: 35 µs one scale per thread, 14 µs here.
+template <bool NARROW>
 __global__ __launch_bounds__(256) void group_scale_vec_kernel(const float* __restrict__ scale,
                                                               int64_t lds, int64_t rows,
                                                               int64_t cols, int64_t g, void* out,
-                                                              int dtype, int64_t ldo, int* flags) {
-  const int64_t j = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+                                                              int dtype, int64_t ldo, int* flags,
+                                                              int rowshift) {
+  // (a whole workgroup on a row: all from the block indices)
+  const int shift = NARROW ? rowshift : 8;
+  const int64_t first = NARROW ? row_first(shift) : blockIdx.y;
+  const int64_t step = NARROW ? row_step(shift) : gridDim.y;
+  const int64_t j = (NARROW ? row_cell(shift) : (int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   int bad = 0;
   if (j < cols) {
     const int64_t k = (uint32_t)j / (uint32_t)g, j0 = k * g;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    for (int64_t r = first; r < rows; r += step) {
       const float4 v = *reinterpret_cast<const float4*>(scale + r * lds + j);
       const float f = scale[r * lds + j0];
       bad |= !(v.x == f) | !(v.y == f) | !(v.z == f) | !(v.w == f);
@@ -164,14 +177,6 @@ bool rows16(const void* p, int64_t ld) {
   return ld % 4 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-// A grid of `cells` threads per row: at most about 16384 workgroups in all.
-dim3 row_grid(int64_t cells, int64_t rows) {
-  const int64_t gx = cdiv(cells, (int64_t)256);
-  return dim3((unsigned)gx, (unsigned)std::max<int64_t>(
-                                1, std::min<int64_t>(std::min<int64_t>(rows, 65535),
-                                                     cdiv((int64_t)16384, gx))));
-}
-
 unsigned grid_of(int64_t n) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdiv(n, 256), 16384));
 }
@@ -209,10 +214,16 @@ extern "C" int g2ptq_pack_quantized(void* stream, const float* codes, int64_t ld
   G2PTQ_CHECK(codes && packed && ldc >= cols && ldp >= words, "pack_quantized: bad codes/packed");
   hipStream_t st = as_stream(stream);
   const bool whole = cols % pf == 0 && rows16(codes, ldc) && words < (1ll << 31);
-  const dim3 pgrid = row_grid(words, rows);
-#define G2_PACK(PF)                                                                          \
-  hipLaunchKernelGGL(pack_codes_vec_kernel<PF>, pgrid, dim3(256), 0, st, codes, ldc, rows,   \
-                     bits, packed, ldp, words)
+  const RowLaunch pl = row_launch(words, rows);
+#define G2_PACK(PF)                                                                           \
+  do {                                                                                        \
+    if (pl.shift < 8)                                                                         \
+      hipLaunchKernelGGL((pack_codes_vec_kernel<PF, true>), pl.grid, dim3(256), 0, st, codes, \
+                         ldc, rows, bits, packed, ldp, words, pl.shift);                      \
+    else                                                                                      \
+      hipLaunchKernelGGL((pack_codes_vec_kernel<PF, false>), pl.grid, dim3(256), 0, st,       \
+                         codes, ldc, rows, bits, packed, ldp, words, pl.shift);               \
+  } while (0)
   if (whole && pf == 4) G2_PACK(4);
   else if (whole && pf == 8) G2_PACK(8);
   else if (whole && pf == 16) G2_PACK(16);
@@ -227,10 +238,15 @@ extern "C" int g2ptq_pack_quantized(void* stream, const float* codes, int64_t ld
                     ldo >= cols / groupsize,
                 "pack_quantized: group size %lld must divide %lld columns", (long long)groupsize,
                 (long long)cols);
-    if (groupsize % 4 == 0 && rows16(scale, lds) && cols < (1ll << 31))
-      hipLaunchKernelGGL(group_scale_vec_kernel, row_grid(cols / 4, rows), dim3(256), 0, st, scale,
-                         lds, rows, cols, groupsize, scale_out, dtype, ldo, flags);
-    else
+    if (groupsize % 4 == 0 && rows16(scale, lds) && cols < (1ll << 31)) {
+      const RowLaunch sl = row_launch(cols / 4, rows);
+      if (sl.shift < 8)
+        hipLaunchKernelGGL(group_scale_vec_kernel<true>, sl.grid, dim3(256), 0, st, scale, lds,
+                           rows, cols, groupsize, scale_out, dtype, ldo, flags, sl.shift);
+      else
+        hipLaunchKernelGGL(group_scale_vec_kernel<false>, sl.grid, dim3(256), 0, st, scale, lds,
+                           rows, cols, groupsize, scale_out, dtype, ldo, flags, sl.shift);
+    } else
       hipLaunchKernelGGL(group_scale_kernel, dim3(grid_of(rows * cols)), dim3(256), 0, st, scale,
                          lds, rows, cols, groupsize, scale_out, dtype, ldo, flags);
     G2PTQ_LAUNCHED();
