@@ -171,8 +171,11 @@ extern "C" int g2ptq_group_mean_square(void* stream, const void* x, int dtype, i
   hipStream_t st = as_stream(stream);
   const float inv_gs = 1.0f / (float)gs;
   // 16-byte loads where every group starts on a 16-byte boundary and holds
-  // whole steps of eight values.
-  if (gs % 8 == 0 && ldx % 8 == 0 && aligned16(x)) {
+  // whole steps of eight values, from groups of 128 on: narrower ones leave
+  // most of a wave's lanes without a step (8192 rows of 4096 bf16, one value
+  // per lane and load against eight: groups of 32 148 and 181 µs, of 64 78 and
+  // 93, of 128 51 and 48, of 256 38 and 25).
+  if (gs >= 128 && gs % 8 == 0 && ldx % 8 == 0 && aligned16(x)) {
     if (dtype == 0)
       hipLaunchKernelGGL(group_mean_square_vec_kernel<uint16_t>, grid, dim3(256), 0, st,
                          static_cast<const uint16_t*>(x), rows, ldx, groups, gs, inv_gs, out);

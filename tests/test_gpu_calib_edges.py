@@ -30,6 +30,20 @@ def test_group_mean_square(dev, dtype, rows, groups, gs, offset):
 
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("gs", [8, 16, 32, 64, 120])
+def test_narrow_groups_take_one_value_per_lane(dev, dtype, gs):
+    """Groups under 128 values, where eight per lane are slower: the same sums in
+    the same order as off the 16-byte grid, bit for bit."""
+    from g2ptq_amd.calib_utils import group_mean_square
+    print(f"narrow groups of {gs} {dtype}", flush=True)
+    x = torch.randn(33 * 4 * gs, generator=gen(gs)).to(dtype).to(dev)
+    off = torch.empty(x.numel() + 1, dtype=dtype, device=dev)[1:]
+    off.copy_(x)
+    assert torch.equal(group_mean_square(x.view(33, 4 * gs), 4),
+                       group_mean_square(off.view(33, 4 * gs), 4))
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("n,offset", [(8, 0), (24, 0), (7, 0), (4096, 0), (4097, 0), (4096, 1)])
 def test_running_mean(dev, dtype, n, offset):
     from g2ptq_amd.calib_utils import running_mean_update
