@@ -136,8 +136,8 @@ __global__ __launch_bounds__(256) void find_params_kernel(const float* __restric
 // A symmetric grid has one scale per distinct max(|xmin1|, xmax1): the
 // 2·steps values that occur stand for all steps² candidates, each with its
 // first position in the scan.  Rows outside the bounds' range (zero, tiny,
-// huge or non-finite groups, other norms, more than kMseCand candidates) scan
-// every candidate exactly.  The first pass costs about 37 cycles per wave and
+// huge or non-finite groups, other norms, more than kMseCand candidates or only
+// a few) scan every candidate exactly.  The first pass costs about 37 cycles per wave and
 // element (six VALU operations and two transcendental ones).  MI355X, groups
 // of 128: 131072 groups, 625 asymmetric candidates 39.5 -> 3.03 ms; 2048
 // groups, symmetric 970 -> 19 us (the exhaustive scan it replaces on the
@@ -214,8 +214,10 @@ __global__ __launch_bounds__(256) void find_params_mse_kernel(const float* __res
                                                               int64_t ldp, int* flags) {
   __shared__ float lower_s[4][kMseCand];
   __shared__ float shrink[kMseSteps];
-  for (int i = threadIdx.x; i < steps && i < kMseSteps; i += 256) shrink[i] = mse_shrink(i, grid);
-  __syncthreads();
+  if (steps > 1) {  // the bracketing pass's factors
+    for (int i = threadIdx.x; i < steps && i < kMseSteps; i += 256) shrink[i] = mse_shrink(i, grid);
+    __syncthreads();
+  }
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t row = (int64_t)blockIdx.x * 4 + wave;
@@ -284,9 +286,16 @@ __global__ __launch_bounds__(256) void find_params_mse_kernel(const float* __res
   const int ncand = listed ? 2 * steps : steps * steps;
   const float p = hr ? 2.f : norm;
   const float vmax = fmaxf(fabsf(mn), fabsf(mx));
+  // Few candidates are scanned exactly at once: the bracketing pass takes a whole
+  // wave's time per 64 of them, however few there are.  4096 groups of 128,
+  // MI355X, µs scanned and bracketed: 1 candidate 6.4 and 16.7, 4 13 and 18, 9
+  // 26 and 18; with weights (no pow) 9 14 and 16, 16 21 and 16; groups of 16: 4
+  // 9.5 and 7.7, with weights 7.7 and 8.4, 9 11 and 8.4.
+  const int few = hr ? (cols >= 64 ? 9 : 4) : (cols >= 64 ? 4 : 1);
   // The bounds hold for scales in [2^-24, 2^24] and |t| <= 2^10 (no overflow
   // and no harmful underflow of d^p in the exact pass), 1 <= p <= 3.
-  bool bounded = nan == 0 && h_ok && positive && ncand <= kMseCand && p >= 1.f && p <= 3.f &&
+  bool bounded = (int64_t)steps * steps > few && nan == 0 && h_ok && positive &&
+                 ncand <= kMseCand && p >= 1.f && p <= 3.f &&
                  vmax > 0.f && vmax < 0x1p34f && cols <= (1 << 20) &&
                  (!hr || hsum >= 0x1p-60f * (float)cols);
   if (bounded) {

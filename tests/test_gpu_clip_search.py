@@ -46,3 +46,39 @@ def test_selected_candidates_equal_exhaustive_scan(dev, rows, cols, bits, grid, 
     assert torch.equal(s * 2.0 ** -30, s30)
     assert torch.equal(z.nan_to_num(nan=99.0), z30.nan_to_num(nan=99.0))
     assert f == f30
+
+
+@pytest.mark.parametrize("cols,steps,sym,weighted", [
+    (128, 1, True, False), (128, 1, False, True), (512, 1, False, False), (16, 1, True, False),
+    (128, 2, False, False), (512, 2, True, False), (128, 3, True, True), (512, 3, False, True)])
+def test_few_candidates_take_no_longer_than_the_scan(dev, cols, steps, sym, weighted):
+    """A search of a few candidates is not bracketed first: it takes what the
+    rows above the bounds' range take, which are scanned (bracketing made it 1.2
+    to 5 times)."""
+    from g2ptq_amd import _core, _lib
+    rows = (1 << 23) // max(cols, 64)
+    g = gen(cols + steps)
+    x = (torch.randn(rows, cols, generator=g) * 0.02).to(dev)
+    h = (torch.rand(1, cols, generator=g) + 0.1).to(dev) if weighted else None
+    s, z = torch.empty(rows, device=dev), torch.empty(rows, device=dev)
+    flags = torch.zeros(1, dtype=torch.int32, device=dev)
+
+    def us(v, n=20):
+        best = float("inf")
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(n):
+                _lib.call("g2ptq_find_params_mse", _core.stream(), _lib.ptr(v), rows, cols, cols, 4,
+                          int(sym), 2.0, 10, (steps + 0.5) / 10, _lib.ptr(h), cols,
+                          1 if weighted else 0, 1, _lib.ptr(s), _lib.ptr(z), 1, _lib.ptr(flags))
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) / n * 1e3)
+        return best
+    huge = x * 2.0 ** 42
+    assert huge.abs().amax(1).min() >= 2.0 ** 34  # no row can be bracketed
+    search, scan = us(x), us(huge)
+    print(f"{steps}x{steps} candidates, groups of {cols}, sym={sym} weighted={weighted}: "
+          f"{search:.1f} us, the scan {scan:.1f} us", flush=True)
+    assert search <= 1.15 * scan
