@@ -46,48 +46,92 @@ __device__ __forceinline__ float row_lane(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + O, 0xf, 0xf, true));
 }
 
-// c −= bcast(mp, lane C of each row)·m, one fused multiply-add with the
-// broadcast on its operand (the compiler keeps a separate v_mov_b32_dpp).  A
-// DPP operand needs two wait states after the VALU write of its register:
-// FIRST carries them for a pivot's mp and orders the other uses behind it
-// (the compiler sees no hazard inside inline assembly; operands that come from
-// LDS need none).
-template <int C, bool FIRST>
-__device__ __forceinline__ void row_fma(float& c, float& mp, float m) {
-  if constexpr (FIRST)
-    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(c), "+v"(mp) : "v"(m), "n"(C));
-  else
-    asm("v_fmac_f32_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
-        : "+v"(c) : "v"(mp), "v"(m), "n"(C));
+// A DPP operand needs two wait states after the VALU write of its register, the
+// result of a reciprocal root one before another VALU instruction reads it, and
+// the compiler sees neither inside inline assembly, nor is it known which copies
+// and reloads it puts before one.  So what belongs together is one statement,
+// which nothing can be put into, and which waits for its operands itself.  (The
+// broadcasts are operands of the multiply-adds: the compiler keeps a separate
+// v_mov_b32_dpp for each.  One statement per multiply-add, the operands' waits
+// left to chance, was no faster: the factor of 2048 columns takes 0.71 ms either way.)
+#define G2_COLS(c)                                                                              \
+  "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5]), "+&v"(c[6]),    \
+      "+&v"(c[7]), "+&v"(c[8]), "+&v"(c[9]), "+&v"(c[10]), "+&v"(c[11]), "+&v"(c[12]),          \
+      "+&v"(c[13]), "+&v"(c[14]), "+&v"(c[15])
+#define G2_FMA(reg, k, q, b, m)                                                                \
+  ".if " #k " >= %" #q "\n\tv_fmac_f32_dpp %" #reg ", %" #b ", -%" #m " row_newbcast:" #k        \
+  " row_mask:0xf bank_mask:0xf\n\t.endif\n\t"
+
+// c[k] −= bcast(b, lane k of each row)·m for k = Q, …, 15.
+template <int Q>
+__device__ __forceinline__ void row_fma(float (&c)[PB], float b, float m) {
+  static_assert(PB == 16, "one entry per lane of a row");
+#define G2_K(k) G2_FMA(k, k, 18, 16, 17)
+  if constexpr (Q < PB)
+    asm("s_nop 1\n\t"
+        G2_K(0) G2_K(1) G2_K(2) G2_K(3) G2_K(4) G2_K(5) G2_K(6) G2_K(7) G2_K(8) G2_K(9) G2_K(10)
+        G2_K(11) G2_K(12) G2_K(13) G2_K(14) G2_K(15)
+        : G2_COLS(c)
+        : "v"(b), "v"(m), "n"(Q));
+#undef G2_K
 }
 
-// The panel's columns C, C + 1, … after pivot J with multipliers m (the
-// lane's row) and mp (the diagonal block's row).
-template <int J, int C>
-__device__ __forceinline__ void pot_update(float (&a)[PB], float (&p)[PB], float m, float& mp) {
-  if constexpr (C < PB) {
-    row_fma<C, C == J + 1>(p[C], mp, mp);
-    row_fma<C, false>(a[C], mp, m);
-    pot_update<J, C + 1>(a, p, m, mp);
-  }
+// Pivot J of a panel, whose reciprocal root is rd: the multipliers mp of the
+// lane's row of the diagonal block and m of its own row, and the update of the
+// columns J + 1, …, the block's (p) before the row's (a); between the two the
+// next pivot dn and its reciprocal root rdn, which takes its time beside a's
+// updates.  (A wait of two states: m's product and one more, the block's updates
+// after p[J + 1]'s, a's updates.)
+template <int J>
+__device__ __forceinline__ void pot_update(float (&p)[PB], float (&a)[PB], float rd, float& m,
+                                           float& dn, float& rdn) {
+  float mp;
+#define G2_M(k, reg)                                                                           \
+  ".if " #k " == %38\n\tv_mul_f32 %34, %" #k ", %36\n\tv_mul_f32 %35, %" #reg ", %36\n\t.endif\n\t"
+#define G2_P(k) G2_FMA(k, k, 37, 34, 34)
+#define G2_D(k)                                                                                \
+  ".if " #k " == %37\n\tv_mov_b32_dpp %32, %" #k " row_newbcast:" #k                            \
+  " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t.endif\n\t"
+#define G2_A(k, reg) G2_FMA(reg, k, 37, 34, 35)
+  asm(".if %38 == 0\n\ts_nop 0\n\t.endif\n\t"  // the first root is the compiler's instruction
+      G2_M(0, 16) G2_M(1, 17) G2_M(2, 18) G2_M(3, 19) G2_M(4, 20) G2_M(5, 21) G2_M(6, 22)
+      G2_M(7, 23) G2_M(8, 24) G2_M(9, 25) G2_M(10, 26) G2_M(11, 27) G2_M(12, 28) G2_M(13, 29)
+      G2_M(14, 30)
+      "s_nop 0\n\t"
+      G2_P(1) G2_P(2) G2_P(3) G2_P(4) G2_P(5) G2_P(6) G2_P(7) G2_P(8) G2_P(9) G2_P(10) G2_P(11)
+      G2_P(12) G2_P(13) G2_P(14) G2_P(15)
+      ".if %37 > 13\n\ts_nop 1\n\t.endif\n\t"
+      G2_D(1) G2_D(2) G2_D(3) G2_D(4) G2_D(5) G2_D(6) G2_D(7) G2_D(8) G2_D(9) G2_D(10) G2_D(11)
+      G2_D(12) G2_D(13) G2_D(14) G2_D(15)
+      "v_rsq_f32 %33, %32\n\t"
+      G2_A(1, 17) G2_A(2, 18) G2_A(3, 19) G2_A(4, 20) G2_A(5, 21) G2_A(6, 22) G2_A(7, 23)
+      G2_A(8, 24) G2_A(9, 25) G2_A(10, 26) G2_A(11, 27) G2_A(12, 28) G2_A(13, 29) G2_A(14, 30)
+      G2_A(15, 31)
+      : G2_COLS(p), G2_COLS(a), "=&v"(dn), "=&v"(rdn), "=&v"(mp), "=&v"(m)
+      : "v"(rd), "n"(J + 1), "n"(J));
+#undef G2_M
+#undef G2_P
+#undef G2_D
+#undef G2_A
 }
+#undef G2_FMA
+#undef G2_COLS
 
-// A panel's pivot J and the ones after it: lane i holds row i's panel columns
-// in a, and row k0 + i % 16's (of the panel's diagonal block) in p.
+// A panel's pivot J (d, its reciprocal root rd) and the ones after it: lane i
+// holds row i's panel columns in a, and row k0 + i % 16's (of the panel's
+// diagonal block) in p.
 template <int J>
 __device__ __forceinline__ void pot_pivots(float (&a)[PB], float (&p)[PB], float (&l)[PB],
-                                           float& rdl, float& dl, int i) {
+                                           float& rdl, float& dl, int i, float d, float rd) {
   if constexpr (J < PB) {
-    const float d = row_lane<J>(p[J]);
-    const float rd = __builtin_amdgcn_rsqf(d);
-    float mp = p[J] * rd;
-    const float m = a[J] * rd;
-    l[J] = m;
     rdl = (i == J) ? rd : rdl;
     dl = (i == J) ? d : dl;
-    pot_update<J, J + 1>(a, p, m, mp);
-    pot_pivots<J + 1>(a, p, l, rdl, dl, i);
+    float dn = 0.f, rdn = 0.f;
+    if constexpr (J + 1 < PB)
+      pot_update<J>(p, a, rd, l[J], dn, rdn);
+    else
+      l[J] = a[J] * rd;
+    pot_pivots<J + 1>(a, p, l, rdl, dl, i, dn, rdn);
   }
 }
 
@@ -102,7 +146,8 @@ __device__ __forceinline__ void pot_panel(const float* As, float* Lm, float* rdv
   for (int c = 0; c < PB; ++c) p[c] = As[(k0 + (i & 15)) * XP + k0 + c];
 #pragma unroll
   for (int c = 0; c < PB; ++c) a[c] = As[i * XP + k0 + c];
-  pot_pivots<0>(a, p, l, rdl, dl, i);
+  const float d = row_lane<0>(p[0]);
+  pot_pivots<0>(a, p, l, rdl, dl, i, d, __builtin_amdgcn_rsqf(d));
 #pragma unroll
   for (int c4 = 0; c4 < PB; c4 += 4)
     *reinterpret_cast<float4*>(&Lm[i * LP + k0 + c4]) = make_float4(l[c4], l[c4 + 1], l[c4 + 2], l[c4 + 3]);
@@ -160,15 +205,6 @@ __device__ __forceinline__ void pot_load_l(float (&l)[PB], const float* Lm, int 
   }
 }
 
-// acc[q] −= l_q·x for q >= Q, l_q on lane q of each row.
-template <int Q>
-__device__ __forceinline__ void pot_axpy(float (&acc)[PB], float& l, float x) {
-  if constexpr (Q < PB) {
-    row_fma<Q, false>(acc[Q], l, x);
-    pot_axpy<Q + 1>(acc, l, x);
-  }
-}
-
 __device__ __forceinline__ void pot_inv_bulk(float (&acc)[PB], const float* Xs, const float* Lm,
                                              int r0, int j0, int i) {
   float l[PB], x[PB];
@@ -176,7 +212,7 @@ __device__ __forceinline__ void pot_inv_bulk(float (&acc)[PB], const float* Xs, 
 #pragma unroll
   for (int j = 0; j < PB; ++j) x[j] = Xs[(j0 + j) * XP + i];
 #pragma unroll
-  for (int j = 0; j < PB; ++j) pot_axpy<0>(acc, l[j], x[j]);
+  for (int j = 0; j < PB; ++j) row_fma<0>(acc, l[j], x[j]);  // l_q on lane q of each row
 }
 
 template <int Q>
@@ -185,7 +221,7 @@ __device__ __forceinline__ void pot_inv_rows(float (&acc)[PB], float (&l)[PB], f
   if constexpr (Q < PB) {
     const float x = acc[Q] * row_lane<Q>(rd);
     X[Q * XP + i] = x;
-    pot_axpy<Q + 1>(acc, l[Q], x);
+    row_fma<Q + 1>(acc, l[Q], x);
     pot_inv_rows<Q + 1>(acc, l, rd, X, i);
   }
 }
