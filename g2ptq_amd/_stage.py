@@ -21,7 +21,7 @@ that are not bf16 take P bf16 planes for Xᵀ that sum to it exactly (fp16: 2,
 fp32: 3; the reference's ``inp.float()``, gptq_utils.py:125), and the
 weighted kind then stages the hi/lo parts of (x·s[t,g])ᵀ as planes; a Gram
 product sums over the pairs of its operands' planes.  GPTQ's fp16 activations
-are staged and multiplied as fp16, one product as for bf16.
+are staged and multiplied as fp16, one plane and one product as for bf16.
 The library gives each layout's height
 (``g2ptq_hessian_stage_height``).
 
@@ -80,10 +80,8 @@ KIND_GPTQ, KIND_GPTAQ, KIND_WEIGHTED = 0, 1, 2
 _GRAM_WS = {KIND_GPTQ: "g2ptq_hessian_gram_workspace",
             KIND_GPTAQ: "g2ptq_gptaq_gram_workspace",
             KIND_WEIGHTED: "g2ptq_weighted_gram_workspace"}
-# activation dtype codes of the any-dtype entry points, and the bf16 planes
-# each stages for Xᵀ
+# activation dtype codes of the any-dtype entry points
 DTYPE_BF16, DTYPE_F16, DTYPE_F32 = 0, 1, 2
-_X_PLANES = {DTYPE_BF16: 1, DTYPE_F16: 2, DTYPE_F32: 3}
 
 
 def _ceil(x, m):
@@ -138,7 +136,7 @@ class GramStager:
         self.kind = kind
         self.G = groups
         self.dtype = dtype
-        # rows of staged bf16 per token column
+        # rows of staged 16-bit elements per token column
         self.height = _lib.query_size_i64("g2ptq_hessian_stage_height", kind, dtype, columns,
                                           groups if kind == KIND_WEIGHTED else 0)
         budget = budget_bytes if budget_bytes is not None else DEFAULT_BUDGET

@@ -1123,7 +1123,7 @@ GramPlan wplan(int64_t K, int64_t C, int64_t G) {
 // Feature planes (Cp rows) staged per kind (0 Hessian, 1 GPTAQ, 2 weighted
 // with G groups) for an activation of P planes.
 int64_t kind_planes(int kind, int64_t G, int P = 1) {
-  if (fused_weighted(kind, P)) return 1;
+  if (fused_weighted(kind, P) || native16(kind, P)) return 1;
   return P + (kind == 1 ? 2 : kind == 2 ? 2 * G : 0);
 }
 
@@ -1315,7 +1315,7 @@ int gram_kind(hipStream_t st, int kind, uint16_t* XT, int64_t ldt, int64_t K, in
   const int64_t width = kind_width(kind, K, C, P, G);
   G2PTQ_CHECK(width <= ldt, "hessian gram: staged operand too narrow (%lld < %lld)",
               (long long)ldt, (long long)width);
-  G2PTQ_TRY(zero_pad(st, XT, ldt, (native16(kind, P) ? 1 : kind_planes(kind, G, P)) * Cp, K, width));
+  G2PTQ_TRY(zero_pad(st, XT, ldt, kind_planes(kind, G, P) * Cp, K, width));
   if (fused_weighted(kind, P)) {
     // the weight rows, as 2G rows of 2·ldt bf16 elements
     G2PTQ_TRY(zero_pad(st, XT + plane, 2 * ldt, G, 2 * K, 2 * width));

@@ -184,10 +184,10 @@ int g2ptq_weighted_gram(void* stream, uint16_t* XT, int64_t ldt, int64_t K, int6
  * the kind's planes as above (GPTAQ: hi, lo of X_fp − X; weighted with
  * P > 1: hi, lo of x·S[t,g]·s_scale per group; weighted bf16: the weight
  * rows of g2ptq_weighted_stage); the plain Hessian of fp16 activations stages
- * them as they are in the first of its two planes and leaves the second
- * alone.  g2ptq_hessian_stage_planes gives the count of feature planes
- * (rows × ldt each) and g2ptq_hessian_stage_height the buffer's height in
- * rows of ldt bf16 (planes × rows, plus the bf16 weighted kind's 2G).
+ * them as they are, one plane of fp16.  g2ptq_hessian_stage_planes gives the
+ * count of feature planes (rows × ldt each) and g2ptq_hessian_stage_height the
+ * buffer's height in rows of ldt 16-bit elements (planes × rows, plus the bf16
+ * weighted kind's 2G).
  * g2ptq_hessian_gram_ex sums each product over the pairs of row and column
  * planes: one fp16 product for the plain Hessian of fp16, the pairs above
  * 2⁻²³ of the product for fp32 (6 of 9; 5 of 6 for GPTAQ's cross term and

@@ -66,16 +66,17 @@ def test_size_queries(lib):
             > _lib.query_size("g2ptq_weighted_gram_workspace", 32768, 4096, 1) > 0)
     rows = _lib.query_size_i64("g2ptq_hessian_stage_rows", 4096)
     assert rows >= 4096 and rows % 256 == 0
-    # any-dtype staging: Xᵀ takes 1 / 2 / 3 bf16 planes for bf16 / fp16 / fp32
+    # any-dtype staging: Xᵀ takes 1 / 2 / 3 bf16 planes for bf16 / fp16 / fp32, and one
+    # plane of fp16 where fp16 is multiplied as it is (the plain Hessian)
     planes = lambda kind, dt, G=0: _lib.query_size_i64("g2ptq_hessian_stage_planes", kind, dt, G)
-    assert [planes(0, dt) for dt in (0, 1, 2)] == [1, 2, 3]
+    assert [planes(0, dt) for dt in (0, 1, 2)] == [1, 1, 3]
     assert [planes(1, dt) for dt in (0, 1, 2)] == [3, 4, 5]
     assert [planes(2, dt, 4) for dt in (0, 1, 2)] == [1, 10, 11]
     # buffer heights in rows of bf16: planes × rows, and the bf16 weighted
     # kind's G fp32 weight rows (2G bf16 rows)
     height = lambda kind, dt, G=0: _lib.query_size_i64("g2ptq_hessian_stage_height", kind, dt,
                                                        4096, G)
-    assert [height(0, dt) for dt in (0, 1, 2)] == [rows, 2 * rows, 3 * rows]
+    assert [height(0, dt) for dt in (0, 1, 2)] == [rows, rows, 3 * rows]
     assert height(1, 0) == 3 * rows
     assert [height(2, dt, 4) for dt in (0, 1, 2)] == [rows + 8, 10 * rows, 11 * rows]
     ex = lambda kind, dt: _lib.query_size("g2ptq_hessian_gram_ex_workspace", kind, dt, 32768, 4096,
