@@ -350,6 +350,7 @@ struct G2Args {
   int64_t tiles;   // upper triangle nt (nt + 1) / 2, or nt² for full products
   int64_t C;
   int S;           // splits (parts × splits per part)
+  bool tree;       // symmetric products: their splits are added in pairs
   int parts;
   float alpha, beta;
   float* H; int64_t ldh;
@@ -872,9 +873,10 @@ __global__ __launch_bounds__(NTH) void wgram_kernel(G2Args a) {
       I, J, diag, wm, wn, lh, lr);
 }
 
-// sum[k] += a thread's row k (16 rows apart) of N consecutive splits, in split
-// order, all of them loaded first.
-template <int N>
+// sum[k] += a thread's row k (16 rows apart) of N consecutive splits, all of them
+// loaded first: one after the other, or (TREE) added in pairs before they reach
+// the sum, which rounds a quarter as often at its full size.
+template <int N, bool TREE>
 __device__ __forceinline__ void reduce_splits(float4 (&sum)[4], const float* p0) {
   float4 p[N][4];
 #pragma unroll
@@ -882,13 +884,29 @@ __device__ __forceinline__ void reduce_splits(float4 (&sum)[4], const float* p0)
 #pragma unroll
     for (int k = 0; k < 4; ++k)
       p[u][k] = *reinterpret_cast<const float4*>(p0 + u * (int64_t)(TT * TT) + 16 * k * TT);
+  auto add = [](float4& d, const float4& e) { d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w; };
+  if constexpr (TREE) {
 #pragma unroll
-  for (int u = 0; u < N; ++u)
+    for (int h = 1; h < N; h *= 2)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      sum[k].x += p[u][k].x; sum[k].y += p[u][k].y;
-      sum[k].z += p[u][k].z; sum[k].w += p[u][k].w;
-    }
+      for (int u = 0; u + h < N; u += 2 * h)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) add(p[u][k], p[u + h][k]);
+  }
+#pragma unroll
+  for (int u = 0; u < (TREE ? 1 : N); ++u)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) add(sum[k], p[u][k]);
+}
+template <bool TREE>
+__device__ __forceinline__ void reduce_all(float4 (&sum)[4], const float* p0, int S) {
+  int sp = 0;
+  for (; sp + 4 <= S; sp += 4) reduce_splits<4, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
+  if (S & 2) {
+    reduce_splits<2, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
+    sp += 2;
+  }
+  if (S & 1) reduce_splits<1, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
 }
 
 // H[I,J] = beta·H + alpha·Σ_s partial_s (fixed order), mirrored for symmetric
@@ -928,13 +946,8 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) sum[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   if (!FULL) {
-    int sp = 0;
-    for (; sp + 4 <= a.S; sp += 4) reduce_splits<4>(sum, p0 + sp * (int64_t)(TT * TT));
-    if (a.S & 2) {
-      reduce_splits<2>(sum, p0 + sp * (int64_t)(TT * TT));
-      sp += 2;
-    }
-    if (a.S & 1) reduce_splits<1>(sum, p0 + sp * (int64_t)(TT * TT));
+    if (a.tree) reduce_all<true>(sum, p0, a.S);
+    else reduce_all<false>(sum, p0, a.S);
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -997,8 +1010,8 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
 // operand has `planes` planes: the smallest power of two that gives at least
 // 4096 workgroups (16 waves of one 256×256 tile per CU) for one column plane,
 // at most 16 splits of one column plane in all and at least 16 KS-token stages
-// per split; then, among the
-// counts down to three quarters of it, the one whose grid fills its last wave
+// per split (twice that count for a `fine` product of more than one step); then,
+// among the counts down to three quarters of it, the one whose grid fills its last wave
 // of workgroups best (one workgroup per CU, kCUs of them): C=4096 has 136
 // tiles, 2176 workgroups (8.5 waves) at 16 splits and 2040 (7.97) at 15, and
 // its Gram takes 4.25 instead of 4.49 ms; C=14336 keeps 4 splits (6384
@@ -1016,17 +1029,19 @@ constexpr int64_t kCUs = 256;  // MI355X
 // Share of the workgroup slots that a grid of n workgroups keeps busy over its waves.
 double wave_fill(int64_t n) { return (double)n / (double)(cdiv(n, kCUs) * kCUs); }
 
-GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, int64_t max_chain = 0,
-                   int64_t max_s = 16) {
+GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, bool fine = false,
+                   int64_t max_chain = 0, int64_t max_s = 16) {
   const int64_t K1 = std::max<int64_t>(K, 1);
   const int64_t smax =
       std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(16 / planes, max_s), K1 / (KS * 16)));
   int s = 1;
   while (s * 2 <= smax && tiles * planes * s < 4096) s *= 2;
+  const int64_t grid1 = fine ? tiles : tiles * planes;  // workgroups per split
+  if (fine && K1 > 2 * KS) s *= 2;
   {
     int best = s;
     for (int c = s - 1; c >= 1 && 4 * c >= 3 * s; --c)
-      if (wave_fill(tiles * planes * c) > wave_fill(tiles * planes * best) + 1e-9) best = c;
+      if (wave_fill(grid1 * c) > wave_fill(grid1 * best) + 1e-9) best = c;
     s = best;
   }
   while (max_chain > 0 && s * 2 <= smax && cdiv(K1, s) > max_chain) s *= 2;
@@ -1055,8 +1070,7 @@ int dtype_planes(int dtype) { return dtype == 0 ? 1 : dtype == 1 ? 2 : 3; }
 // plane, exact products, one MFMA where the two bf16 planes take four (they
 // remain for GPTAQ's and the weighted operands, whose second factor is not an
 // fp16 value).  C = 4096, 32768 tokens, MI355X: products 2188 -> 609 us, reduces
-// 336 -> 155, staging 236 -> 131; rms distance from fp64 (of
-// sqrt(H_ii·H_jj), C = 4096, 16384 tokens) 3.0e-9 -> 2.8e-9.
+// 336 -> 155, staging 236 -> 131.
 bool native16(int kind, int P) { return kind == 0 && P == 2; }
 
 // A product: Σ over pairs (row plane, column plane) of staged planes, counted
@@ -1066,6 +1080,8 @@ struct Product {
   int planes;                 // the row operand's planes: set the split count (error of a chain)
   int parts;
   int a[kMaxParts], b[kMaxParts];
+  bool fine = false;          // twice the splits (products of 22 significant bits)
+  bool tree = false;          // partial sums added in pairs
 };
 // X's P planes against themselves, H = Σ X_pᵀX_q (upper tiles of each pair,
 // which is exact for the symmetric sum), smallest pairs first.  An fp32 value
@@ -1089,15 +1105,22 @@ Product v_product(int P, bool full) {
   p.full = full;
   return p;
 }
-Product h_product(int kind, int P) { return native16(kind, P) ? X1 : x_product(P); }
+// fp16 as it is: one pair, at twice the splits that the two bf16 planes had and
+// with its partial sums added in pairs.  Its products have 22 significant bits
+// where a bf16 pair's have 16, and chains as long as theirs round more: rms
+// distance from fp64, of that of the two planes' sums, 0.47 to 0.92 between 2000
+// and 32768 tokens at C = 700 to 5120 (at the planes' splits 0.56 to 1.17); the
+// same time (C = 4096, 16384 tokens 0.68 ms, C = 1000, 3000 tokens 79 -> 69 us).
+constexpr Product N1{false, 2, 1, {0}, {0}, true, true};
+Product h_product(int kind, int P) { return native16(kind, P) ? N1 : x_product(P); }
 
 size_t product_ws(int64_t K, int64_t C, Product pr) {
   const int64_t tiles = n_tiles(C, pr.full);
-  return plan_ws_bytes(tiles, gram_plan(tiles, K, pr.planes, pr.parts));
+  return plan_ws_bytes(tiles, gram_plan(tiles, K, pr.planes, pr.parts, pr.fine));
 }
 
 int64_t product_width(int64_t K, int64_t C, Product pr) {
-  return gram_plan(n_tiles(C, pr.full), K, pr.planes, pr.parts).Kp;
+  return gram_plan(n_tiles(C, pr.full), K, pr.planes, pr.parts, pr.fine).Kp;
 }
 
 // The weighted kind of bf16 activations runs all G groups in one
@@ -1117,7 +1140,7 @@ constexpr int64_t kWBudget = int64_t(16) << 30;
 GramPlan wplan(int64_t K, int64_t C, int64_t G) {
   const int64_t items = n_tiles(C, false) * G;
   const int64_t max_s = std::max<int64_t>(1, kWBudget / (items * TT * TT * 4));
-  return gram_plan(items, K, 1, 1, kWChain, max_s);
+  return gram_plan(items, K, 1, 1, false, kWChain, max_s);
 }
 
 // Feature planes (Cp rows) staged per kind (0 Hessian, 1 GPTAQ, 2 weighted
@@ -1172,7 +1195,7 @@ int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint
                 float* out, int64_t ldo, void* ws, size_t ws_bytes, bool f16 = false) {
   const int64_t nt = cdiv(C, TT);
   const int64_t tiles = n_tiles(C, pr.full);
-  const GramPlan p = gram_plan(tiles, K, pr.planes, pr.parts);
+  const GramPlan p = gram_plan(tiles, K, pr.planes, pr.parts, pr.fine);
   G2PTQ_CHECK(p.Kp <= ldt, "hessian gram: staged operand too narrow (%lld < %lld)",
               (long long)ldt, (long long)p.Kp);
   G2PTQ_CHECK(tiles * p.S < (1ll << 31) && tiles < 65536, "hessian gram: grid too large");
@@ -1183,7 +1206,7 @@ int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint
     a.B[q] = B + pr.b[q] * plane;
   }
   a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
-  a.S = p.S; a.parts = pr.parts; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
+  a.S = p.S; a.parts = pr.parts; a.tree = pr.tree; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
   a.G = 1;
   if (p.S > 1) {
     const size_t need = plan_ws_bytes(tiles, p);

@@ -37,3 +37,29 @@ def test_gram_of_fp16_and_fp32_tokens(dev, dtype, C, T, size):
     print(f"max normalized error {err:.3g}, bound {bound:.3g}", flush=True)
     assert err <= bound
     assert torch.equal(H, H.t())
+
+
+@pytest.mark.parametrize("C,T", [(700, 2000), (1100, 2000), (700, 8000), (2752, 14000)])
+def test_fp16_products_are_no_less_exact_than_plane_pairs(dev, C, T):
+    """GPTAQ's H of the same fp16 tokens is the sum over the pairs of two bf16
+    planes; the rms distance of GPTQ's from fp64 is no larger (over four inputs,
+    of sqrt(H_ii·H_jj))."""
+    from g2ptq_amd import GPTAQ, GPTQ
+    print(f"fp16 against plane pairs C={C} T={T}", flush=True)
+    off = {"gptq": 0.0, "gptaq": 0.0}
+    for seed in range(4):
+        g = torch.Generator(device=dev).manual_seed(100 * seed + C)
+        X = (torch.randn(T, C, device=dev, generator=g)
+             * torch.exp(torch.randn(C, device=dev, generator=g))).half()
+        He = X.double().t().mm(X.double())
+        d = torch.diagonal(He)
+        for name in off:
+            lin = torch.nn.Linear(C, 4, bias=False).to(dev)
+            m = GPTQ([lin]) if name == "gptq" else GPTAQ([lin])
+            if name == "gptaq":
+                m.fp_inp[0] = [X]
+            m.add_batch(0, X.unsqueeze(0), None)
+            err = (m.H[0].double() / 2 - He) / torch.sqrt(d[:, None] * d[None, :])
+            off[name] += err.pow(2).mean().item()
+    print(f"rms distance squared: fp16 {off['gptq']:.3g}, pairs {off['gptaq']:.3g}", flush=True)
+    assert off["gptq"] <= off["gptaq"]
