@@ -336,8 +336,8 @@ __global__ void zero_cols_bf16_kernel(uint16_t* XT, int64_t ldt, int64_t rows, i
     XT[(e / w) * ldt + k0 + (e % w)] = 0;
 }
 
-// Most plane pairs a product sums over (fp32 activations: kXParts below).
-constexpr int kMaxParts = 6;
+// Most plane pairs a product sums over (fp32 activations, X3 below).
+constexpr int kMaxParts = 9;
 
 struct G2Args {
   // The product is Σ over `parts` pairs of planes (row operand A[p], column
@@ -350,7 +350,6 @@ struct G2Args {
   int64_t tiles;   // upper triangle nt (nt + 1) / 2, or nt² for full products
   int64_t C;
   int S;           // splits (parts × splits per part)
-  bool tree;       // symmetric products: their splits are added in pairs
   int parts;
   float alpha, beta;
   float* H; int64_t ldh;
@@ -874,46 +873,54 @@ __global__ __launch_bounds__(NTH) void wgram_kernel(G2Args a) {
 }
 
 // sum[k] += a thread's row k (16 rows apart) of N consecutive splits, all of them
-// loaded first: one after the other, or (TREE) added in pairs before they reach
-// the sum, which rounds a quarter as often at its full size.
-template <int N, bool TREE>
-__device__ __forceinline__ void reduce_splits(float4 (&sum)[4], const float* p0) {
-  float4 p[N][4];
+// loaded first: in split order, or (TREE) added in pairs before they reach the
+// sum, which rounds a quarter as often at its full size.
+template <int N, bool TREE, int R = 4>
+__device__ __forceinline__ void reduce_splits(float4 (&sum)[R], const float* p0) {
+  float4 p[N][R];
 #pragma unroll
   for (int u = 0; u < N; ++u)
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < R; ++k)
       p[u][k] = *reinterpret_cast<const float4*>(p0 + u * (int64_t)(TT * TT) + 16 * k * TT);
-  auto add = [](float4& d, const float4& e) { d.x += e.x; d.y += e.y; d.z += e.z; d.w += e.w; };
   if constexpr (TREE) {
+    __builtin_amdgcn_sched_barrier(0);  // else the loads are put off to their pair's turn
 #pragma unroll
     for (int h = 1; h < N; h *= 2)
 #pragma unroll
       for (int u = 0; u + h < N; u += 2 * h)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) add(p[u][k], p[u + h][k]);
+        for (int k = 0; k < R; ++k) {
+          p[u][k].x += p[u + h][k].x; p[u][k].y += p[u + h][k].y;
+          p[u][k].z += p[u + h][k].z; p[u][k].w += p[u + h][k].w;
+        }
   }
 #pragma unroll
   for (int u = 0; u < (TREE ? 1 : N); ++u)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) add(sum[k], p[u][k]);
+    for (int k = 0; k < R; ++k) {
+      sum[k].x += p[u][k].x; sum[k].y += p[u][k].y;
+      sum[k].z += p[u][k].z; sum[k].w += p[u][k].w;
+    }
 }
-template <bool TREE>
-__device__ __forceinline__ void reduce_all(float4 (&sum)[4], const float* p0, int S) {
+
+// The R rows of a thread, all splits.
+template <bool TREE, int R>
+__device__ __forceinline__ void reduce_rows(float4 (&sum)[R], const float* p0, int S) {
   int sp = 0;
-  for (; sp + 4 <= S; sp += 4) reduce_splits<4, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
+  for (; sp + 4 <= S; sp += 4) reduce_splits<4, TREE, R>(sum, p0 + sp * (int64_t)(TT * TT));
   if (S & 2) {
-    reduce_splits<2, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
+    reduce_splits<2, TREE, R>(sum, p0 + sp * (int64_t)(TT * TT));
     sp += 2;
   }
-  if (S & 1) reduce_splits<1, TREE>(sum, p0 + sp * (int64_t)(TT * TT));
+  if (S & 1) reduce_splits<1, TREE, R>(sum, p0 + sp * (int64_t)(TT * TT));
 }
 
 // H[I,J] = beta·H + alpha·Σ_s partial_s (fixed order), mirrored for symmetric
 // products.  One workgroup reduces a 64×64 block of a tile: rows are read and
 // written as 16-byte vectors, and the mirror goes through an LDS transpose so
 // that it is written in rows as well.
-template <bool FULL>
+template <bool FULL, bool TREE>
 __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
   __shared__ float tr[64][65];
   const int64_t tile = blockIdx.y, grp = blockIdx.z;  // grp: weighted products' group
@@ -945,14 +952,15 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
   float4 sum[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) sum[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (!FULL) {
-    if (a.tree) reduce_all<true>(sum, p0, a.S);
-    else reduce_all<false>(sum, p0, a.S);
-  }
+  if (!FULL) reduce_rows<TREE, 4>(sum, p0, a.S);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int r = r0 + 16 * k;  // row within the block
-    if (FULL) {
+    if (FULL && TREE) {
+      float4 row[1] = {sum[k]};
+      reduce_rows<true, 1>(row, p0 + 16 * k * TT, a.S);
+      sum[k] = row[0];
+    } else if (FULL) {
       for (int sp = 0; sp < a.S; ++sp) {
         const float4 p =
             *reinterpret_cast<const float4*>(p0 + sp * (int64_t)(TT * TT) + 16 * k * TT);
@@ -1084,21 +1092,23 @@ struct Product {
   bool tree = false;          // partial sums added in pairs
 };
 // X's P planes against themselves, H = Σ X_pᵀX_q (upper tiles of each pair,
-// which is exact for the symmetric sum), smallest pairs first.  An fp32 value
-// is three planes of 8 significant bits: the pairs (1, 2), (2, 1) and (2, 2)
-// are below 2⁻²³ of the product and left out (the others sum to the product
-// of two 24-bit values within fp32's own rounding: rms distance from fp64 at
-// C = 2752, 14000 tokens 4.4e-9 of sqrt(H_ii·H_jj), with all nine pairs
-// 4.7e-9).  All pairs run in one launch: products 1175 -> 714 us, reduces
-// 154 -> 100 (MI355X, that size).
+// which is exact for the symmetric sum), smallest pairs first, all in one
+// launch.  An fp32 value is three planes of 8 significant bits, and every pair
+// counts: (1, 2) and (2, 1) are up to 2⁻²⁴ of the product each, and left out
+// (C = 4096, 16384 tokens: 1.97 ms instead of 2.90) they put tokens whose planes
+// all have one sign off by a further 0.6 to 1.2e-7 of H.  One launch with the
+// partial sums added in pairs against a launch per column plane: rms distance
+// from fp64 0.56 to 0.99 of theirs between 1000 and 32768 tokens at C = 257 to
+// 5120; C = 2752, 14000 tokens 1540 -> 1350 us.
 constexpr Product X1{false, 1, 1, {0}, {0}};
-constexpr Product X2{false, 2, 4, {1, 1, 0, 0}, {1, 0, 1, 0}};
-constexpr Product X3{false, 3, 6, {2, 0, 1, 1, 0, 0}, {0, 2, 1, 0, 1, 0}};
+constexpr Product X2{false, 2, 4, {1, 1, 0, 0}, {1, 0, 1, 0}, false, true};
+constexpr Product X3{false, 3, 9, {2, 2, 1, 2, 0, 1, 1, 0, 0}, {2, 1, 2, 0, 2, 1, 0, 1, 0}, false,
+                     true};
 // The two planes (hi, lo) of a 16-bit operand against X's P planes: GPTAQ's
-// (X_fp − X) and the weighted x·w.  (lo, 2) is below 2⁻²³ and left out.
+// (X_fp − X) and the weighted x·w.
 constexpr Product V1{false, 2, 2, {0, 1}, {0, 0}};
-constexpr Product V2{false, 2, 4, {1, 0, 1, 0}, {1, 1, 0, 0}};
-constexpr Product V3{false, 2, 5, {0, 1, 0, 1, 0}, {2, 1, 1, 0, 0}};
+constexpr Product V2{false, 2, 4, {1, 0, 1, 0}, {1, 1, 0, 0}, false, true};
+constexpr Product V3{false, 2, 6, {1, 0, 1, 0, 1, 0}, {2, 2, 1, 1, 0, 0}, false, true};
 Product x_product(int P) { return P == 1 ? X1 : P == 2 ? X2 : X3; }
 Product v_product(int P, bool full) {
   Product p = P == 1 ? V1 : P == 2 ? V2 : V3;
@@ -1206,7 +1216,7 @@ int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint
     a.B[q] = B + pr.b[q] * plane;
   }
   a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
-  a.S = p.S; a.parts = pr.parts; a.tree = pr.tree; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
+  a.S = p.S; a.parts = pr.parts; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
   a.G = 1;
   if (p.S > 1) {
     const size_t need = plan_ws_bytes(tiles, p);
@@ -1228,10 +1238,15 @@ int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint
   }
   G2PTQ_LAUNCHED();
   if (p.S > 1) {
-    if (pr.full)
-      hipLaunchKernelGGL(gram_reduce_kernel<true>, dim3(16, (unsigned)tiles), dim3(256), 0, st, a);
+    const dim3 rgrid(16, (unsigned)tiles);
+    if (pr.full && pr.tree)
+      hipLaunchKernelGGL((gram_reduce_kernel<true, true>), rgrid, dim3(256), 0, st, a);
+    else if (pr.full)
+      hipLaunchKernelGGL((gram_reduce_kernel<true, false>), rgrid, dim3(256), 0, st, a);
+    else if (pr.tree)
+      hipLaunchKernelGGL((gram_reduce_kernel<false, true>), rgrid, dim3(256), 0, st, a);
     else
-      hipLaunchKernelGGL(gram_reduce_kernel<false>, dim3(16, (unsigned)tiles), dim3(256), 0, st, a);
+      hipLaunchKernelGGL((gram_reduce_kernel<false, false>), rgrid, dim3(256), 0, st, a);
     G2PTQ_LAUNCHED();
   }
   return G2PTQ_OK;
@@ -1267,7 +1282,7 @@ int run_wproduct(hipStream_t st, const uint16_t* XT, const float* W, int64_t ldw
   else hipLaunchKernelGGL(wgram_kernel<false>, grid, dim3(NTH), 0, st, a);
   G2PTQ_LAUNCHED();
   if (p.S > 1) {
-    hipLaunchKernelGGL(gram_reduce_kernel<false>, dim3(16, (unsigned)tiles, (unsigned)G), dim3(256),
+    hipLaunchKernelGGL((gram_reduce_kernel<false, false>), dim3(16, (unsigned)tiles, (unsigned)G), dim3(256),
                        0, st, a);
     G2PTQ_LAUNCHED();
   }

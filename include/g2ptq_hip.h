@@ -188,11 +188,11 @@ int g2ptq_weighted_gram(void* stream, uint16_t* XT, int64_t ldt, int64_t K, int6
  * count of feature planes (rows × ldt each) and g2ptq_hessian_stage_height the
  * buffer's height in rows of ldt 16-bit elements (planes × rows, plus the bf16
  * weighted kind's 2G).
- * g2ptq_hessian_gram_ex sums each product over the pairs of row and column
- * planes: one fp16 product for the plain Hessian of fp16, the pairs above
- * 2⁻²³ of the product for fp32 (6 of 9; 5 of 6 for GPTAQ's cross term and
- * the weighted kind).  The updates are those of g2ptq_hessian_gram,
- * g2ptq_gptaq_gram and g2ptq_weighted_gram, whose bf16 paths these equal bit
+ * g2ptq_hessian_gram_ex sums each product over all pairs of row and column
+ * planes: one fp16 product for the plain Hessian of fp16, nine pairs for that
+ * of fp32, six for fp32's GPTAQ cross term and weighted kind.  The updates are
+ * those of g2ptq_hessian_gram, g2ptq_gptaq_gram and g2ptq_weighted_gram, whose
+ * bf16 paths these equal bit
  * for bit.  Same alignment and padding rules as g2ptq_hessian_stage / _gram;
  * act (kind 2) as in g2ptq_weighted_stage. */
 int g2ptq_hessian_stage_planes(int kind, int dtype, int64_t G, int64_t* planes);

@@ -3,7 +3,8 @@ like bf16 (``inp.float()``, gptq_utils/gptq_utils.py:125, gptaq_utils.py:
 139-146, g2ptq_utils.py:193-201, gptq_guided_utils.py:59-81).
 
 The HIP path stages such an activation as bf16 planes that sum to it exactly
-(fp16: 2, fp32: 3) and runs every Gram product once per plane.  Each case
+(fp16: 2, fp32: 3) and sums every Gram product over all pairs of its operands'
+planes; a plain Hessian's fp16 tokens are multiplied as they are.  Each case
 accumulates the Hessians from the same tokens as the oracle (fp32 on the
 host), holds them to fp64 sums of the same tokens (1e-5 relative to
 sqrt(H_ii·H_jj)), and holds the whole flow to oracle.parity.check_flow.
