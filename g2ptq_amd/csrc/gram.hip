@@ -1019,8 +1019,8 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
 // 4096 workgroups (16 waves of one 256×256 tile per CU) for one column plane,
 // at most 16 splits of one column plane in all and at least 16 KS-token stages
 // per split (twice that count for a `fine` product of more than one step); then,
-// among the counts down to three quarters of it, the one whose grid fills its last wave
-// of workgroups best (one workgroup per CU, kCUs of them): C=4096 has 136
+// among the counts down to three quarters of it, the one whose grid fills its last
+// wave of workgroups best (one workgroup per CU, kCUs of them): C=4096 has 136
 // tiles, 2176 workgroups (8.5 waves) at 16 splits and 2040 (7.97) at 15, and
 // its Gram takes 4.25 instead of 4.49 ms; C=14336 keeps 4 splits (6384
 // workgroups, 24.9 waves).  Measured on MI355X with random bf16 operands.
@@ -1033,6 +1033,7 @@ struct GramPlan {
 };
 
 constexpr int64_t kCUs = 256;  // MI355X
+constexpr int64_t kMaxPartials = 4096;  // more of them (1 GiB) only where a chain needs them
 
 // Share of the workgroup slots that a grid of n workgroups keeps busy over its waves.
 double wave_fill(int64_t n) { return (double)n / (double)(cdiv(n, kCUs) * kCUs); }
@@ -1050,6 +1051,25 @@ GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, bool fine = 
     int best = s;
     for (int c = s - 1; c >= 1 && 4 * c >= 3 * s; --c)
       if (wave_fill(grid1 * c) > wave_fill(grid1 * best) + 1e-9) best = c;
+    s = best;
+  }
+  // A product of several pairs launches `parts` times the tiles: of the counts
+  // from there to a quarter (or one) more, with at least 8 KS-token stages per
+  // split (its chains grow no longer), the one that takes the least, in tokens of
+  // a full round of workgroups: their rounds, and writing and reading their
+  // partials (about 4 tokens each; small grids reduce slower, so no further).  MI355X, fp32 tokens, with the launch taken for tiles·planes
+  // workgroups and here: C = 768, 4000 tokens 132 -> 116 us, C = 1280, 20000 tokens
+  // 593 -> 540.
+  if (parts > 1 && parts != planes) {
+    auto cost = [&](int64_t c) {
+      const int64_t step = (int64_t)2 * KS * c;
+      return cdiv(tiles * parts * c, kCUs) * (cdiv(K1, step) * step / c) + 4 * tiles * parts * c;
+    };
+    const int64_t most = std::min<int64_t>(std::min<int64_t>(16 / planes, K1 / (KS * 8)),
+                                           s + std::max(1, s / 4));
+    int best = s;
+    for (int c = s + 1; c <= most && tiles * parts * c <= kMaxPartials; ++c)
+      if (cost(c) < cost(best)) best = c;
     s = best;
   }
   while (max_chain > 0 && s * 2 <= smax && cdiv(K1, s) > max_chain) s *= 2;

@@ -1,0 +1,39 @@
+"""CPU: the split counts of Hessians of several planes fit the launch they make.
+
+A product over several pairs of planes launches one workgroup per tile, pair and
+split.  From the workspace that a Gram asks for (a 256x256 fp32 tile per
+workgroup) the count per pair is read back.  `per_plane` is the count that fits
+one launch per column plane best: the one taken is no lower (chains no longer),
+and takes no more tokens, in full rounds of 256 workgroups of which each partial
+tile counts as four, than that or one more.
+"""
+import pytest
+
+from g2ptq_amd import _lib
+
+PAIRS = {(0, 2): (9, 5), (1, 1): (4, 8), (2, 2): (6, 8)}  # pairs, most splits
+
+
+def _cost(tiles, pairs, K, s):
+    tokens = -(-K // (128 * s)) * 128
+    groups = tiles * pairs * s
+    return -(-groups // 256) * tokens + 4 * groups
+
+
+@pytest.mark.parametrize("kind,dtype,C,K,per_plane", [
+    (0, 2, 700, 1100, 1), (0, 2, 700, 2000, 1), (0, 2, 768, 4000, 2), (0, 2, 1280, 20000, 4),
+    (0, 2, 2048, 8192, 4), (0, 2, 2752, 14000, 4), (0, 2, 4096, 16384, 3), (1, 1, 700, 2000, 1),
+    (1, 1, 1000, 3000, 2), (1, 1, 2752, 14000, 8), (2, 2, 768, 4000, 2), (2, 2, 1000, 3000, 2),
+    (2, 2, 2048, 8192, 7)])
+def test_split_count_fits_all_pairs(kind, dtype, C, K, per_plane):
+    pairs, most = PAIRS[kind, dtype]
+    nt = -(-C // 256)
+    tiles = nt * nt if kind == 1 else nt * (nt + 1) // 2  # GPTAQ's cross term asks for the most
+    size = _lib.query_size("g2ptq_hessian_gram_ex_workspace", kind, dtype, K, C,
+                           1 if kind == 2 else 0)
+    s = size // (tiles * pairs * 256 * 256 * 4)
+    assert size == tiles * pairs * s * 256 * 256 * 4
+    assert per_plane <= s <= most
+    for c in (per_plane, per_plane + 1):
+        if c <= min(most, K // 512):
+            assert _cost(tiles, pairs, K, s) <= _cost(tiles, pairs, K, c), (s, c)
