@@ -25,9 +25,12 @@
 // for small grids); each wave a quadrant made of 32×32 MFMA blocks.  K advances
 // in slabs of 32 through double-buffered LDS with 16-byte global loads for
 // two slabs in flight, interleaved with the MFMAs of the current slab.  Large
-// split products with B given N×K (a grid of at least 256 tiles of 256×256,
+// split products with B given N×K (a grid of at least 256 tiles of 256×256
+// that fills its rounds of workgroups about as well as 128×128 tiles would,
 // K >= 384) take an 8-wave 256×256 workgroup instead, which halves the LDS
-// reads and barriers per MFMA and sums the same products in the same order.
+// reads and barriers per MFMA and sums the same products in the same order;
+// long products with few rows keep 128×128 tiles where 64×64 ones would have
+// more workgroups (gemm_f32 has both rules).
 //
 // Operand layout: a 32x32x2 MFMA takes one k per lane half, so a slab's k
 // order is permuted: for k-octet o, lane half h holds k = 8o + 4h + j in the
@@ -156,10 +159,15 @@ struct BoolTag {
 
 // Byte offset from row r0 of an operand's row r0 + r (the last of its R rows
 // where that is past it) and column c: below 2³² for r < 256 and ld < 2²²
-// (gemm_f32's VEC).
+// (near_rows).
 __device__ __forceinline__ uint32_t row_offset(int64_t r0, int r, int64_t R, int64_t ld, int c) {
   const int64_t last = R - 1 - r0;
   return (uint32_t)(((r < last ? r : last) * ld + c) * 4);
+}
+
+// Whether 256 rows of both operands lie within 32-bit byte offsets.
+__device__ __forceinline__ bool near_rows(const GemmF32& g) {
+  return g.lda < (1 << 22) && g.ldb < (1 << 22);
 }
 
 // K range of the tile at (m0, n0): triangular operands contribute nothing
@@ -429,7 +437,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   } while (0)
     // Step t: the MMAs of slab t (buffer t % 2), then slab t+1 goes from its
     // register set into the other buffer and that set loads slab t+5.  Slabs
-    // past the end load zeros and skip their MMAs.
+    // past the end (the last one again, or chunks masked at the store) skip
+    // their MMAs.
     // Interleave the step's MFMAs with the next slab's split (VALU), LDS
     // stores and global loads, so one wave's conversions overlap its own
     // matrix-core work instead of waiting behind the whole MFMA burst.
@@ -489,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
       __builtin_amdgcn_sched_barrier(0);
     };
     if (nk > 0) {
-      if (VEC && ((K - klo) & (SK - 1)) == 0) loop(BoolTag<VEC>{});
+      if (VEC && ((K - klo) & (SK - 1)) == 0 && near_rows(g)) loop(BoolTag<VEC>{});
       else loop(BoolTag<false>{});
     }
 #undef GS_LOAD
@@ -500,8 +509,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
 #undef GS_STEP_IN
 #undef GS_PATTERN
   } else {
-    // Slabs are processed in pairs; a trailing odd slab and the prefetches
-    // past the end load zeros (k >= K is masked), which add nothing.
+    // Slabs are processed in pairs; a trailing odd slab's entries past the end
+    // are stored as zeros (k >= K is masked there), which add nothing.
     const int nk = K > klo ? (int)cdiv(K - klo, (int64_t)BK) : 0;
     const int nk2 = (nk + 1) & ~1;
     if (nk2 > 0) {
@@ -721,7 +730,8 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
 
   // Stage t is multiplied out of buffer t&1 while stage t+1 goes from its
   // register set to the other buffer and that set loads stage t+3; stages
-  // past K load zeros and skip their MFMAs.  One barrier per stage.
+  // past K (the last one again, or chunks masked at the store) skip their
+  // MFMAs.  One barrier per stage.
   auto loop = [&](auto inner_tag) __attribute__((always_inline)) {
     constexpr bool INNER = decltype(inner_tag)::value;
     S2_LOAD(x, 0);
@@ -747,7 +757,7 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  if (VEC && (K & (SK - 1)) == 0) loop(BoolTag<VEC>{});
+  if (VEC && (K & (SK - 1)) == 0 && near_rows(g)) loop(BoolTag<VEC>{});
   else loop(BoolTag<false>{});
 #undef S2_LOAD
 #undef S2_PUT
@@ -861,16 +871,13 @@ int gemm_f32(hipStream_t stream, const GemmF32& g) {
   };
   // ... and whole 16-byte chunks along k (and along n for B given K×N).
   const bool vec = al(g.A, g.lda, g.sA, g.sA2) && al(g.B, g.ldb, g.sB, g.sB2) && g.K % 4 == 0 &&
-                   (g.b_kcontig || g.N % 4 == 0) && g.lda < (1 << 22) && g.ldb < (1 << 22);
+                   (g.b_kcontig || g.N % 4 == 0);
   // 128×128 tiles unless that grid would leave most of the 256 CUs (two
   // workgroups each) idle.
   // Products with K >= 128 run on the bf16 matrix cores from split operands
   // (about 1.3x the fp32 MFMA rate, and no less accurate); the short-K updates
   // of the factor's panels are latency-bound and keep the fp32 MFMAs.
   const bool split = g.K >= 128;
-  G2PTQ_CHECK(!split || g.b_kcontig || g.ldb < (1ll << 27),
-              "gemm_f32: ldb %lld too large for the split path's 32-bit row offsets",
-              (long long)g.ldb);
   const int64_t t256 = cdiv(g.M, (int64_t)S2T) * cdiv(g.N, (int64_t)S2T);
   // 256×256 tiles (one workgroup per CU) against 128×128 (two): the larger
   // tile is 6 to 10 % faster per full round of workgroups, so it is taken

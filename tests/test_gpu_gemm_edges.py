@@ -46,3 +46,35 @@ def test_products_ignore_what_lies_outside(dev, M, N, K, pad, b_trans):
     print(f"max err / |A||B| {err:.3g}", flush=True)
     assert err <= 4e-7
     assert torch.all(D[:, N] == 7.0)
+
+
+@pytest.mark.parametrize("b_trans,lda,ldb", [(1, 1 << 22, 1 << 22), (1, (1 << 22) + 1, 256),
+                                             (0, 1 << 22, 1 << 23), (0, 256, 1 << 27)])
+def test_rows_far_apart(dev, b_trans, lda, ldb):
+    """Pitches past 32-bit offsets within a tile give the packed operands' bits."""
+    from g2ptq_amd import _core, _lib
+    M, N, K = 66, 68, 144
+    span = 4 * (M * lda + (N if b_trans else K) * ldb)
+    if torch.cuda.mem_get_info(dev)[0] < 1.25 * span:
+        pytest.skip("not enough free device memory")
+    print(f"gemm rows {lda} and {ldb} apart, b_trans={b_trans}", flush=True)
+    g = gen(7)
+    A, B = torch.randn(M, K, generator=g).to(dev), torch.randn(N, K, generator=g).to(dev)
+    if not b_trans:
+        B = B.t().contiguous()
+    out = []
+    for far in (False, True):
+        if far:
+            Af = torch.empty(M * lda, device=dev).as_strided((M, K), (lda, 1))
+            Bf = torch.empty(B.shape[0] * ldb, device=dev).as_strided(B.shape, (ldb, 1))
+            Af.copy_(A)
+            Bf.copy_(B)
+            A, B = Af, Bf
+        D = torch.empty(M, N, device=dev)
+        _lib.call("g2ptq_gemm_f32", _core.stream(), M, N, K, 1, _lib.ptr(A), A.stride(0), 0,
+                  _lib.ptr(B), B.stride(0), 0, b_trans, None, 0, 0, _lib.ptr(D), N, 0, 1.0, 0.0)
+        out.append(D)
+    torch.cuda.synchronize()
+    del A, B, Af, Bf
+    torch.cuda.empty_cache()
+    assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
