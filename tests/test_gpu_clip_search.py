@@ -4,7 +4,8 @@ Rows whose scales lie outside [2^-24, 2^24] scan every candidate exactly.  With
 norm 2 (and with Hessian-diagonal weights) the error of a row scaled by 2^-30
 is the row's error scaled by 2^-60, so the search on the scaled rows, which
 takes the exhaustive scan, must return the same zero points and the scales
-times 2^-30, bit for bit.
+times 2^-30, bit for bit.  At other norms the parameters found are held to the
+least error over all candidates, evaluated in fp64.
 """
 import pytest
 import torch
@@ -82,3 +83,58 @@ def test_few_candidates_take_no_longer_than_the_scan(dev, cols, steps, sym, weig
     print(f"{steps}x{steps} candidates, groups of {cols}, sym={sym} weighted={weighted}: "
           f"{search:.1f} us, the scan {scan:.1f} us", flush=True)
     assert search <= 1.15 * scan
+
+
+def _candidates(x, bits, sym, grid, steps):
+    """Scale and zero (rows, 1) of every candidate, formed in fp32 as the search
+    forms them (divisors as tensors: torch multiplies by a number's reciprocal)."""
+    half = 2 ** (bits - 1)
+    xmin, xmax = x.amin(1, keepdim=True).clamp_max(0), x.amax(1, keepdim=True).clamp_min(0)
+    for i in range(steps):
+        for j in range(steps):
+            lo, hi = (1 - i / grid) * xmin, (1 - j / grid) * xmax
+            if sym:
+                s = torch.maximum(lo.abs(), hi) / torch.full_like(lo, (2 * half - 1) / 2)
+                yield s, torch.zeros_like(s)
+            else:
+                s = (hi - lo) / torch.full_like(lo, 2 * half - 1)
+                yield s, torch.clamp(torch.round(-half - lo / s), -half, half - 1)
+
+
+def _error(x, s, z, bits, norm):
+    """Σ|x̂ − x|^norm of a candidate: its fp32 differences, raised and summed in fp64."""
+    half = 2 ** (bits - 1)
+    d = s * (torch.clamp(torch.round(x / s) + z, -half, half - 1) - z) - x
+    return d.double().abs().pow(norm).sum(1, keepdim=True)
+
+
+@pytest.mark.parametrize("sym", [True, False])
+@pytest.mark.parametrize("norm", [0.99, 1.0, 1.7, 2.4, 3.0, 3.01])
+@pytest.mark.parametrize("rows,cols,bits,grid,shrink", [
+    (64, 128, 4, 50, 0.5),      # the scripts' search
+    (64, 16, 2, 50, 0.5), (64, 100, 8, 50, 0.5), (5, 6000, 4, 50, 0.5),
+    (32, 128, 8, 36, 0.89),     # values up to 920 steps of the smallest scale
+    (16, 1000, 3, 32, 1.0)])
+def test_the_best_candidate_is_found(dev, rows, cols, bits, grid, shrink, norm, sym):
+    from g2ptq_amd import WeightQuantizer
+    print(f"clip search {rows}x{cols} W{bits} norm={norm} sym={sym} grid={grid}", flush=True)
+    g = gen(int(100 * norm) + rows + cols)
+    x = torch.randn(rows, cols, generator=g) * 0.02
+    x[0, 0] = 0.3
+    x[1] = x[1].abs()
+    x[2] = -x[2].abs()
+    x[3] = torch.round(x[3] * 200) / 64
+    x = x.to(dev)
+    q = WeightQuantizer()
+    q.configure(bits, perchannel=True, sym=sym, mse=True, norm=norm, grid=grid, maxshrink=shrink)
+    q.find_params(x)
+    found = _error(x, q.scale, q.zero, bits, norm)
+    least = torch.full_like(found, float("inf"))
+    for s, z in _candidates(x, bits, sym, grid, int(shrink * grid)):
+        least = torch.minimum(least, _error(x, s, z, bits, norm))
+    # both the found and the best candidate's fp32 sums are off by at most a chain of
+    # cols / 64 + 6 additions and the rounding of the power
+    slack = 2 * (cols / 64 + 6 + 4) * 2.0 ** -24
+    worst = ((found - least) / least.clamp_min(1e-300)).max().item()
+    print(f"error above the least: {worst:.3g} of it, allowed {slack:.3g}", flush=True)
+    assert torch.all(found - least <= slack * least)
