@@ -1057,7 +1057,9 @@ GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, bool fine = 
   // from there to a quarter (or one) more, with at least 8 KS-token stages per
   // split (its chains grow no longer), the one that takes the least, in tokens of
   // a full round of workgroups: their rounds, and writing and reading their
-  // partials (about 4 tokens each; small grids reduce slower, so no further).  MI355X, fp32 tokens, with the launch taken for tiles·planes
+  // partials (about 4 tokens each; small grids reduce slower, so no further);
+  // within 1/64 the larger, whose chains round less (C = 2752, 14000 fp32 tokens:
+  // 5 for 4, rms distance from fp64 3.8e-9 for 4.4e-9).  MI355X, fp32 tokens, with the launch taken for tiles·planes
   // workgroups and here: C = 768, 4000 tokens 132 -> 116 us, C = 1280, 20000 tokens
   // 593 -> 540.
   if (parts > 1 && parts != planes) {
@@ -1069,7 +1071,7 @@ GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, bool fine = 
                                            s + std::max(1, s / 4));
     int best = s;
     for (int c = s + 1; c <= most && tiles * parts * c <= kMaxPartials; ++c)
-      if (cost(c) < cost(best)) best = c;
+      if (cost(c) <= cost(best) + cost(best) / 64) best = c;
     s = best;
   }
   while (max_chain > 0 && s * 2 <= smax && cdiv(K1, s) > max_chain) s *= 2;

@@ -5,7 +5,8 @@ split.  From the workspace that a Gram asks for (a 256x256 fp32 tile per
 workgroup) the count per pair is read back.  `per_plane` is the count that fits
 one launch per column plane best: the one taken is no lower (chains no longer),
 and takes no more tokens, in full rounds of 256 workgroups of which each partial
-tile counts as four, than that or one more.
+tile counts as four, than that or one more, but for a 64th (where shorter chains
+are as good as free they are taken).
 """
 import pytest
 
@@ -36,4 +37,9 @@ def test_split_count_fits_all_pairs(kind, dtype, C, K, per_plane):
     assert per_plane <= s <= most
     for c in (per_plane, per_plane + 1):
         if c <= min(most, K // 512):
-            assert _cost(tiles, pairs, K, s) <= _cost(tiles, pairs, K, c), (s, c)
+            assert _cost(tiles, pairs, K, s) <= _cost(tiles, pairs, K, c) * 65 // 64, (s, c)
+
+
+def test_near_ties_take_shorter_chains():
+    size = _lib.query_size("g2ptq_hessian_gram_ex_workspace", 0, 2, 14000, 2752, 0)
+    assert size == 66 * 9 * 5 * 256 * 256 * 4  # 12 rounds of 2816 tokens for 10 of 3584
