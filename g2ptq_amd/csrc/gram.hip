@@ -1026,14 +1026,19 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(G2Args a) {
 // workgroups, 24.9 waves).  Measured on MI355X with random bf16 operands.
 // Every split gets an even number of stages, so the staged width is K padded
 // to a multiple of 2·KS·(splits per part), at most 2048.
+// All pairs run in one launch while its partials take at most 3.5 GiB, inside what
+// staging buffers leave free on the device; else as many at a time as the row
+// operand has planes, each launch adding to the output.
 struct GramPlan {
-  int S;        // total splits
+  int S;        // splits of a launch
+  int pairs;    // pairs of a launch
   int64_t Kp;   // padded tokens per part
   int64_t kc;   // tokens per split
 };
 
 constexpr int64_t kCUs = 256;  // MI355X
 constexpr int64_t kMaxPartials = 4096;  // more of them (1 GiB) only where a chain needs them
+constexpr int64_t kMaxOneLaunch = 14336;  // partials of all pairs in one launch (3.5 GiB)
 
 // Share of the workgroup slots that a grid of n workgroups keeps busy over its waves.
 double wave_fill(int64_t n) { return (double)n / (double)(cdiv(n, kCUs) * kCUs); }
@@ -1077,7 +1082,8 @@ GramPlan gram_plan(int64_t tiles, int64_t K, int planes, int parts, bool fine = 
   while (max_chain > 0 && s * 2 <= smax && cdiv(K1, s) > max_chain) s *= 2;
   const int64_t step = (int64_t)2 * KS * s;
   GramPlan p;
-  p.S = s * parts;
+  p.pairs = parts > planes && tiles * parts * s > kMaxOneLaunch ? planes : parts;
+  p.S = s * p.pairs;
   p.Kp = cdiv(K1, step) * step;
   p.kc = p.Kp / s;
   return p;
@@ -1232,44 +1238,48 @@ int run_product(hipStream_t st, const Product& pr, const uint16_t* A, const uint
               (long long)ldt, (long long)p.Kp);
   G2PTQ_CHECK(tiles * p.S < (1ll << 31) && tiles < 65536, "hessian gram: grid too large");
   G2PTQ_CHECK(!f16 || !pr.full, "hessian gram: fp16 planes are for symmetric products");
-  G2Args a{};
-  for (int q = 0; q < pr.parts; ++q) {
-    a.A[q] = A + pr.a[q] * plane;
-    a.B[q] = B + pr.b[q] * plane;
-  }
-  a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
-  a.S = p.S; a.parts = pr.parts; a.alpha = alpha; a.beta = beta; a.H = out; a.ldh = ldo;
-  a.G = 1;
   if (p.S > 1) {
     const size_t need = plan_ws_bytes(tiles, p);
     G2PTQ_CHECK(ws != nullptr && ws_bytes >= need, "hessian gram: workspace %zu < %zu", ws_bytes,
                 need);
+  }
+  for (int q0 = 0; q0 < pr.parts; q0 += p.pairs) {  // each launch after the first adds to out
+    const int n = std::min(p.pairs, pr.parts - q0);
+    G2Args a{};
+    for (int q = 0; q < n; ++q) {
+      a.A[q] = A + pr.a[q0 + q] * plane;
+      a.B[q] = B + pr.b[q0 + q] * plane;
+    }
+    a.ldt = ldt; a.kc = p.kc; a.nt = nt; a.tiles = tiles; a.C = C;
+    a.S = p.S / p.pairs * n; a.parts = n; a.alpha = alpha; a.beta = q0 == 0 ? beta : 1.f;
+    a.H = out; a.ldh = ldo;
+    a.G = 1;
     a.P = static_cast<float*>(ws);
-  }
-  const dim3 grid((unsigned)(tiles * p.S));
-  const bool direct_beta = p.S == 1 && beta != 0.f;
-  if (f16) {
-    if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, false, true>), grid, dim3(NTH), 0, st, a);
-    else hipLaunchKernelGGL((gram256_kernel<false, false, true>), grid, dim3(NTH), 0, st, a);
-  } else if (pr.full) {
-    if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, true>), grid, dim3(NTH), 0, st, a);
-    else hipLaunchKernelGGL((gram256_kernel<false, true>), grid, dim3(NTH), 0, st, a);
-  } else {
-    if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, false>), grid, dim3(NTH), 0, st, a);
-    else hipLaunchKernelGGL((gram256_kernel<false, false>), grid, dim3(NTH), 0, st, a);
-  }
-  G2PTQ_LAUNCHED();
-  if (p.S > 1) {
-    const dim3 rgrid(16, (unsigned)tiles);
-    if (pr.full && pr.tree)
-      hipLaunchKernelGGL((gram_reduce_kernel<true, true>), rgrid, dim3(256), 0, st, a);
-    else if (pr.full)
-      hipLaunchKernelGGL((gram_reduce_kernel<true, false>), rgrid, dim3(256), 0, st, a);
-    else if (pr.tree)
-      hipLaunchKernelGGL((gram_reduce_kernel<false, true>), rgrid, dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL((gram_reduce_kernel<false, false>), rgrid, dim3(256), 0, st, a);
+    const dim3 grid((unsigned)(tiles * a.S));
+    const bool direct_beta = a.S == 1 && a.beta != 0.f;
+    if (f16) {
+      if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, false, true>), grid, dim3(NTH), 0, st, a);
+      else hipLaunchKernelGGL((gram256_kernel<false, false, true>), grid, dim3(NTH), 0, st, a);
+    } else if (pr.full) {
+      if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, true>), grid, dim3(NTH), 0, st, a);
+      else hipLaunchKernelGGL((gram256_kernel<false, true>), grid, dim3(NTH), 0, st, a);
+    } else {
+      if (direct_beta) hipLaunchKernelGGL((gram256_kernel<true, false>), grid, dim3(NTH), 0, st, a);
+      else hipLaunchKernelGGL((gram256_kernel<false, false>), grid, dim3(NTH), 0, st, a);
+    }
     G2PTQ_LAUNCHED();
+    if (a.S > 1) {
+      const dim3 rgrid(16, (unsigned)tiles);
+      if (pr.full && pr.tree)
+        hipLaunchKernelGGL((gram_reduce_kernel<true, true>), rgrid, dim3(256), 0, st, a);
+      else if (pr.full)
+        hipLaunchKernelGGL((gram_reduce_kernel<true, false>), rgrid, dim3(256), 0, st, a);
+      else if (pr.tree)
+        hipLaunchKernelGGL((gram_reduce_kernel<false, true>), rgrid, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((gram_reduce_kernel<false, false>), rgrid, dim3(256), 0, st, a);
+      G2PTQ_LAUNCHED();
+    }
   }
   return G2PTQ_OK;
 }

@@ -87,7 +87,7 @@ def _isolating_columns(dtype, shift):
     return cols, values
 
 
-@pytest.mark.parametrize("C", [8, 300])
+@pytest.mark.parametrize("C", [8, 300, 16500])  # 16500: the pairs in several launches
 @pytest.mark.parametrize("kind", ["gptq", "gptaq", "g2ptq"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
 def test_every_pair_of_planes_counts(dev, dtype, kind, C):
@@ -113,7 +113,14 @@ def test_every_pair_of_planes_counts(dev, dtype, kind, C):
     else:
         m = G2PTQ([lin], [[torch.ones(16, 1)]], [torch.ones(4, C, device=dev)], 1)
     m.add_batch(0, X.unsqueeze(0), None)
-    H = m.H.double().cpu().reshape(C, C)
+    cols = list(range(len(first))) + list(range(at, C))
+
+    def corner(M):
+        """The entries of the isolating columns, at their places."""
+        M = M.reshape(C, C)
+        rows = M[:, cols][cols].double().cpu()
+        return {(i, j): rows[a, b] for a, i in enumerate(cols) for b, j in enumerate(cols)}
+    H = corner(m.H)
     scale = {"gptq": 2.0, "gptaq": 2.0, "g2ptq": 1.0 / 16}[kind]
     # x·w and X_fp − X carry two planes, hi and lo
     rows = range(2 if kind == "g2ptq" else len(values))
@@ -123,7 +130,7 @@ def test_every_pair_of_planes_counts(dev, dtype, kind, C):
             assert abs(H[p, at + q].item() - want) <= 2.0 ** -22 * want, (p, q)
             assert H[at + q, p].item() == H[p, at + q].item(), (q, p)
     if kind == "gptaq":
-        D = m.dXXT.double().cpu().reshape(C, C)
+        D = corner(m.dXXT)
         for p in range(2):
             for q in range(len(values)):
                 want = -scale * 16 * values[p] * values[q]

@@ -43,3 +43,20 @@ def test_split_count_fits_all_pairs(kind, dtype, C, K, per_plane):
 def test_near_ties_take_shorter_chains():
     size = _lib.query_size("g2ptq_hessian_gram_ex_workspace", 0, 2, 14000, 2752, 0)
     assert size == 66 * 9 * 5 * 256 * 256 * 4  # 12 rounds of 2816 tokens for 10 of 3584
+
+
+@pytest.mark.parametrize("kind,dtype,planes", [(0, 1, 2), (0, 2, 3), (1, 1, 2), (1, 2, 2), (2, 1, 2),
+                                               (2, 2, 2)])
+@pytest.mark.parametrize("C", [4096, 5120, 8192, 14336, 28672])
+def test_workspaces_stay_within_what_staging_leaves_free(kind, dtype, planes, C):
+    """Staging buffers leave 4 GiB of the device free: the partials of a Gram take no
+    more than 3.5 of them, or than one launch per column plane takes."""
+    for K in (4096, 16384, 204800):
+        nt = -(-C // 256)
+        tiles = nt * nt if kind == 1 else nt * (nt + 1) // 2
+        size = _lib.query_size("g2ptq_hessian_gram_ex_workspace", kind, dtype, K, C,
+                               1 if kind == 2 else 0)
+        s = 1  # the largest power of two for 4096 workgroups of one column plane
+        while s * 2 <= 16 // planes and tiles * planes * s < 4096:
+            s *= 2
+        assert size <= max(7 << 29, tiles * planes * s * 256 * 256 * 4), (K, size / 2 ** 30)
