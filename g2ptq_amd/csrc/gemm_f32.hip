@@ -244,22 +244,36 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
     return v;
   };
 
-  // Register sets x / y hold one slab each (indices are compile-time constants).
-  float4 xa[RA], xb[RB], ya[RA], yb[RB];
+  // INNER (whole slabs, 16-byte loads, rows within 32-bit offsets): no masks, and
+  // a slab's address is a uniform base plus a 32-bit offset per thread (slabs past
+  // the end re-read the last one and go unused).  Products with B given K×N are
+  // bound by the VALU work between their MFMAs, the split among it, and masks and
+  // 64-bit addresses are a tenth of that: MI355X, 1024×64×2048 57 us with the
+  // masks at the loads, 66 at the stores, 52 here.
 #define GF_LOAD(RAr, RBr, slab)                                                                \
   do {                                                                                         \
-    const int64_t k0_ = klo + (int64_t)(slab) * BK;                                            \
-    _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                          \
-      RAr[i_] = ld4(A, g.lda, m0 + ra_row + 32 * i_, k0_ + ra_kq, M, K);                       \
-    _Pragma("unroll") for (int i_ = 0; i_ < RB; ++i_) {                                        \
-      if (B_KCONTIG) RBr[i_] = ld4(B, g.ldb, n0 + ra_row + 32 * i_, k0_ + ra_kq, N, K);         \
-      else RBr[i_] = ld4(B, g.ldb, k0_ + rb_k + RB_ROWS * i_, n0 + rb_nq, K, N);                \
+    if constexpr (INNER) {                                                                     \
+      const int64_t sl_ = (slab) < nk ? (slab) : nk - 1;                                       \
+      const char* const pa_ = ua + sl_ * (BK * 4);                                             \
+      const char* const pb_ = ub + sl_ * (B_KCONTIG ? BK * 4 : BK * 4 * g.ldb);                \
+      _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                        \
+        RAr[i_] = *reinterpret_cast<const float4*>(pa_ + oa[i_]);                              \
+      _Pragma("unroll") for (int i_ = 0; i_ < RB; ++i_)                                        \
+        RBr[i_] = *reinterpret_cast<const float4*>(pb_ + ob[i_]);                              \
+    } else {                                                                                   \
+      const int64_t k0_ = klo + (int64_t)(slab) * BK;                                          \
+      _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                        \
+        RAr[i_] = ld4(A, g.lda, m0 + ra_row + 32 * i_, k0_ + ra_kq, M, K);                     \
+      _Pragma("unroll") for (int i_ = 0; i_ < RB; ++i_) {                                      \
+        if (B_KCONTIG) RBr[i_] = ld4(B, g.ldb, n0 + ra_row + 32 * i_, k0_ + ra_kq, N, K);       \
+        else RBr[i_] = ld4(B, g.ldb, k0_ + rb_k + RB_ROWS * i_, n0 + rb_nq, K, N);              \
+      }                                                                                        \
     }                                                                                          \
   } while (0)
 #define GF_STORE(RAr, RBr, buf, slab)                                                          \
   do {                                                                                         \
     const int64_t k0_ = klo + (int64_t)(slab) * BK;                                            \
-    const bool ka_ = k0_ + ra_kq < K;                                                          \
+    const bool ka_ = INNER || k0_ + ra_kq < K;                                                 \
     _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                          \
       *reinterpret_cast<float4*>(&As[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) =                \
           keep4(RAr[i_], ka_);                                                                 \
@@ -269,7 +283,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
             keep4(RBr[i_], ka_);                                                               \
       else                                                                                     \
         *reinterpret_cast<float4*>(&Bs[(buf)][(rb_k + RB_ROWS * i_) * PN + rb_nq]) =           \
-            keep4(RBr[i_], k0_ + rb_k + RB_ROWS * i_ < K);                                     \
+            keep4(RBr[i_], INNER || k0_ + rb_k + RB_ROWS * i_ < K);                            \
     }                                                                                          \
   } while (0)
 
@@ -510,31 +524,48 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
 #undef GS_PATTERN
   } else {
     // Slabs are processed in pairs; a trailing odd slab's entries past the end
-    // are stored as zeros (k >= K is masked there), which add nothing.
+    // are stored as zeros (k >= K is masked there), which add nothing, or skipped.
     const int nk = K > klo ? (int)cdiv(K - klo, (int64_t)BK) : 0;
-    const int nk2 = (nk + 1) & ~1;
-    if (nk2 > 0) {
+    uint32_t oa[RA], ob[RB];
+#pragma unroll
+    for (int i = 0; i < RA; ++i) oa[i] = row_offset(m0, ra_row + 32 * i, M, g.lda, ra_kq);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+      ob[i] = B_KCONTIG ? row_offset(n0, ra_row + 32 * i, N, g.ldb, ra_kq)
+                        : (uint32_t)(((rb_k + RB_ROWS * i) * g.ldb +
+                                      (n0 + rb_nq < N ? n0 + rb_nq : 0)) * 4);
+    const char* const ua = reinterpret_cast<const char*>(A + m0 * g.lda + klo);
+    const char* const ub =
+        reinterpret_cast<const char*>(B_KCONTIG ? B + n0 * g.ldb + klo : B + klo * g.ldb);
+    float4 xa[RA], xb[RB], ya[RA], yb[RB];  // one slab each
+    auto loop = [&](auto inner_tag) __attribute__((always_inline)) {
+      constexpr bool INNER = decltype(inner_tag)::value;
       GF_LOAD(xa, xb, 0);
       GF_STORE(xa, xb, 0, 0);
       GF_LOAD(xa, xb, 1);
       GF_LOAD(ya, yb, 2);
-    }
-    __syncthreads();
-    for (int kt = 0; kt < nk2; kt += 2) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (SPLIT) GF_MMA_SPLIT(0); else GF_MMA(0);  // slab kt
-      GF_STORE(xa, xb, 1, kt + 1);
-      GF_LOAD(xa, xb, kt + 3);
-      __builtin_amdgcn_sched_barrier(0);
       __syncthreads();
+      for (int kt = 0; kt < nk; kt += 2) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (SPLIT) GF_MMA_SPLIT(0); else GF_MMA(0);  // slab kt
+        GF_STORE(xa, xb, 1, kt + 1);
+        GF_LOAD(xa, xb, kt + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        if (INNER && kt + 1 >= nk) break;
+        __builtin_amdgcn_sched_barrier(0);
+        if (SPLIT) GF_MMA_SPLIT(1); else GF_MMA(1);  // slab kt+1
+        GF_STORE(ya, yb, 0, kt + 2);
+        GF_LOAD(ya, yb, kt + 4);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+      }
       __builtin_amdgcn_sched_barrier(0);
-      if (SPLIT) GF_MMA_SPLIT(1); else GF_MMA(1);  // slab kt+1
-      GF_STORE(ya, yb, 0, kt + 2);
-      GF_LOAD(ya, yb, kt + 4);
-      __builtin_amdgcn_sched_barrier(0);
-      __syncthreads();
+    };
+    if (nk > 0) {
+      if (VEC && ((K - klo) & (BK - 1)) == 0 && near_rows(g)) loop(BoolTag<VEC>{});
+      else loop(BoolTag<false>{});
     }
-    __builtin_amdgcn_sched_barrier(0);
   }
 #undef GF_LOAD
 #undef GF_STORE

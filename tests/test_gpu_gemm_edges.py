@@ -78,3 +78,29 @@ def test_rows_far_apart(dev, b_trans, lda, ldb):
     del A, B, Af, Bf
     torch.cuda.empty_cache()
     assert torch.equal(out[0].view(torch.int32), out[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 64, 2048), (64, 1024, 4096), (512, 500, 512)])
+def test_small_products_with_b_given_by_rows(dev, M, N, K):
+    """B given K×N, whose fragments every wave splits for itself, takes 1.25 times
+    the N×K product's time where few workgroups run (1.5 with masked loads)."""
+    from g2ptq_amd import _core, _lib
+    A, B = torch.randn(M, K, device=dev), torch.randn(N * K, device=dev)
+    D = torch.empty(M, N, device=dev)
+
+    def us(b_trans, n=30):
+        best = float("inf")
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(n):
+                _lib.call("g2ptq_gemm_f32", _core.stream(), M, N, K, 1, _lib.ptr(A), K, 0,
+                          _lib.ptr(B), K if b_trans else N, 0, b_trans, None, 0, 0, _lib.ptr(D), N,
+                          0, 1.0, 0.0)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) / n * 1e3)
+        return best
+    kn, nk = us(0), us(1)
+    print(f"{M}x{N}x{K}: B by rows {kn:.1f} us, by columns {nk:.1f} us", flush=True)
+    assert kn <= 1.4 * nk
