@@ -225,7 +225,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   // stored to LDS, one to four slabs later: a mask at the load makes the wave
   // wait for memory in the very slab that issues it.  Only k needs a mask:
   // rows (columns) past M (N) are multiplied and never stored.  With VEC a
-  // 16-byte chunk is wholly inside or outside the k range.  MI355X, masks at
+  // 16-byte chunk is wholly inside or outside the k range; without it every
+  // element is tested at its load and no mask is left.  MI355X, masks at
   // the loads before, split products: 512×2048×2048 (64×64 tiles) 61 -> 47 us,
   // 512×8192×8192 (128×128) 522 -> 404, 1024×4096×4096 four times (256×256)
   // 682 -> 644.
@@ -273,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
 #define GF_STORE(RAr, RBr, buf, slab)                                                          \
   do {                                                                                         \
     const int64_t k0_ = klo + (int64_t)(slab) * BK;                                            \
-    const bool ka_ = INNER || k0_ + ra_kq < K;                                                 \
+    const bool ka_ = INNER || !VEC || k0_ + ra_kq < K;                                         \
     _Pragma("unroll") for (int i_ = 0; i_ < RA; ++i_)                                          \
       *reinterpret_cast<float4*>(&As[(buf)][(ra_row + 32 * i_) * PK + ra_kq]) =                \
           keep4(RAr[i_], ka_);                                                                 \
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
             keep4(RBr[i_], ka_);                                                               \
       else                                                                                     \
         *reinterpret_cast<float4*>(&Bs[(buf)][(rb_k + RB_ROWS * i_) * PN + rb_nq]) =           \
-            keep4(RBr[i_], INNER || k0_ + rb_k + RB_ROWS * i_ < K);                            \
+            keep4(RBr[i_], INNER || !VEC || k0_ + rb_k + RB_ROWS * i_ < K);                    \
     }                                                                                          \
   } while (0)
 
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(GemmF32 g, int64_t tm,
   } while (0)
 #define GS_STORE(RA_, RB_, buf, slab)                                                          \
   do {                                                                                         \
-    const bool k_ = INNER || klo + (int64_t)(slab) * SK + sa_kq < K;                           \
+    const bool k_ = INNER || !VEC || klo + (int64_t)(slab) * SK + sa_kq < K;                   \
     _Pragma("unroll") for (int i_ = 0; i_ < RS; ++i_) {                                        \
       const int o_ = (buf) * 3 * PL + (sa_row + 64 * i_) * SP + sa_kq;                         \
       GS_PUT(Ap + o_, keep4(RA_[i_], k_));                                                     \
@@ -717,7 +718,7 @@ __global__ __launch_bounds__(512) void gemm_s256_kernel(GemmF32 g, int64_t tm, i
   } while (0)
 #define S2_STORE(R, buf, st)                                                                   \
   do {                                                                                         \
-    const bool k_ = INNER || (int64_t)(st) * SK + sa_kq < K;                                   \
+    const bool k_ = INNER || !VEC || (int64_t)(st) * SK + sa_kq < K;                           \
     S2_PUT(Ap, buf, sa_row, keep4(R##a0, k_));                                                 \
     S2_PUT(Ap, buf, sa_row + 128, keep4(R##a1, k_));                                           \
     S2_PUT(Bp, buf, sa_row, keep4(R##b0, k_));                                                 \
